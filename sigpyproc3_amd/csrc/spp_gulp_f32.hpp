@@ -1,0 +1,15 @@
+// One-DM dedispersion of a float32 gulp (gulp_f32.hip), called by spp_dedisperse.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace spp {
+
+// out[t] = float32(sum over c of in[t + delays[c]][c] in float64 and channel order), t < nout.
+// Negative rows wrap by nsamps; rows outside the gulp after that read as 0.
+int launch_ded_f32(const float* in, const int32_t* delays, float* out, int64_t nchans, int64_t nsamps, int64_t nout,
+                   hipStream_t st);
+
+}  // namespace spp
