@@ -13,10 +13,12 @@
 // Work per output sample: nchans adds; HBM bytes per gulp: nsamps * nchans * nbits/8
 // read + 4 * nout written. For 1/2-bit data that is under a byte per add, and the kernel is
 // bound by instruction issue (a byte write per sample staged, a byte read and an add per
-// sample summed), not by HBM.
+// sample summed), not by HBM. The subband form combines a band's channel groups by float
+// atomics, about 2e10 per second: 8-bit gulps with many bands go to subband8.hip instead.
 #include "spp_common.hpp"
 #include "spp_gulp_f32.hpp"
 #include "spp_gulp_swar.hpp"
+#include "spp_subband8.hpp"
 #include "spp_unpack.hpp"
 
 #include <algorithm>
@@ -558,6 +560,9 @@ extern "C" int spp_subband(const void* in, int nbits, int big, int64_t nchans, i
         SPP_LAUNCHED("k_subband_f32");
         return SPP_OK;
     }
+    if (nbits == 8 && spp::subband8_applies(in, nchans, nout, nsubs))
+        return spp::launch_subband8(static_cast<const uint8_t*>(in), delays, chan_to_sub, out, nchans, nsamps, nout,
+                                    nsubs, out_size, st);
     return launch_int<1>(static_cast<const uint8_t*>(in), nbits, big, delays, chan_to_sub, out,
                          nchans, nsamps, nout, 0, nsubs, out_size, st);
 }
