@@ -537,8 +537,8 @@ __global__ void k_boxcar_final(const Best* __restrict__ part, int64_t nrows, int
 // ---------------------------------------------------------------- fused normalise + boxcar MF
 //
 // The running normalisation and the boxcar MF of the rows of a plane x in one pass: z never
-// leaves the block. A block takes the RN_CHB outputs of one row that k_norm's block takes, and
-// normalises them RN_SEG at a time with the same window sums and arithmetic (so z is the
+// leaves the block. A block takes `chb` outputs of one row (whole segments) and
+// normalises them RN_SEG at a time with k_norm's window sums and arithmetic (so z is the
 // float32 k_norm writes). Each segment's z is prefix-summed in float64, relative to the block
 // start, into an LDS ring P of two segments; the box sums of the previous segment are then
 // P[u + w] - P[u]. A box reaches wmax - 1 <= MF_WMAX - 1 < RN_SEG samples into the next
@@ -549,8 +549,8 @@ __global__ void k_boxcar_final(const Best* __restrict__ part, int64_t nrows, int
 // Per width the block keeps the first maximum of the box sum over its outputs, and the sum of
 // its z (counted twice for t < Ng - n, the samples that recur in zt[n, Ng)) towards S. The
 // maximum is found in two passes per segment: each lane's largest sum per width (straight
-// reads and float64 max), then exact first-position tracking only in the waves where some
-// lane reaches the largest sum the block has tracked so far -- about one segment in nine
+// reads and float64 max), then the first position of the wave's maximum only in the waves where
+// some lane reaches the largest sum the block has tracked so far -- about one segment in nine
 // after the first, as a new running maximum is rare.
 // k_nb_final adds a row's chunk sums in order, takes each width's first maximum over the
 // chunks, forms conv_w = (box - w S / Ng) / sqrt(w (1 - w / Ng)) in float64, rounds to
@@ -565,7 +565,11 @@ struct NbRow {
 };
 
 constexpr int NB_RING = 2 * RN_SEG;
-constexpr int NB_NONE = 0x3fffffff;   // position code of "no candidate" (codes are < 2^10)
+
+// Ring slots repeated past its end, and samples kept of the row's head: the widest box, in whole
+// runs of a thread's samples.
+__host__ __device__ constexpr int nb_mirror(int wmax) { return (wmax + RN_PER - 1) / RN_PER * RN_PER; }
+constexpr int nb_lds_bytes(int wmax) { return 8 * (NB_RING + nb_mirror(wmax)) + 4 * nb_mirror(wmax); }
 constexpr int NB_NOPOS = 0x7fffffff;  // position of "no candidate" (positions are < 2^31 - 1)
 
 // An unsigned key with the order of the doubles (NaN aside): sign bit set for x >= 0,
@@ -575,23 +579,29 @@ __device__ __forceinline__ unsigned long long order_key(double x) {
     return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
 }
 
-// NWMAX: widths the per-width loops are unrolled for; EXACT: nw == NWMAX (no per-width
-// branch, so the box reads of one width can be in flight while the previous one is reduced).
-// Three blocks per CU (the LDS allows three); two for the 32-width form, whose per-width
-// registers would not fit three.
-template <int NWMAX, bool EXACT, bool ALIGNED>
-__global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
-    const float* __restrict__ x, int64_t ldx, const NbRow* __restrict__ rows, int64_t nb_row,
+// One kernel for any number of widths: nothing is kept per width in registers. Each wave's
+// first maximum per width lives in LDS and is touched only when pass 2 runs; the widths and the
+// block's tracked maxima sit in one VGPR each, lane wi holding width wi's, and are read by
+// v_readlane. (Holding every lane's own maximum cost 3 VGPRs per width: at 14 widths 65 spilled
+// of 256 and 301 x 160007 samples took 625 us; now 320.) The LDS is sized for the widest box, so
+// that four blocks share a CU up to 512 samples: 1024 x 2^19 samples, 9 widths, 2.33 -> 2.09 ms
+// against three. Bound by VALU issue (102 operations per output, 65 % busy) and the barriers of
+// each segment's scans.
+template <bool ALIGNED>
+__global__ __launch_bounds__(RN_THREADS, 4) void k_norm_boxcar(
+    const float* __restrict__ x, int64_t ldx, const NbRow* __restrict__ rows, int64_t nb_row, int64_t chb,
     int64_t nblocks, int32_t window, const int32_t* __restrict__ widths, int nw, int32_t wmax,
     double* __restrict__ part_s, double* __restrict__ part_v, int32_t* __restrict__ part_t) {
-    __shared__ double ring[NB_RING + MF_WMAX];
-    __shared__ float head[RN_SEG];
+    extern __shared__ __align__(16) double ring[];  // NB_RING + nmirror values, then head
+    const int nmirror = nb_mirror(wmax);
+    float* __restrict__ head = reinterpret_cast<float*>(ring + NB_RING + nmirror);  // z[0, nmirror)
     __shared__ double sa[RN_THREADS / 64], sb[RN_THREADS / 64], red[RN_THREADS / 64];
     // per width: the upper 32 bits of the order key (order_key) of the largest box sum any lane
     // of the block has tracked so far
-    __shared__ uint32_t tau_hi[NWMAX];
-    __shared__ double wv[NWMAX][RN_THREADS / 64];
-    __shared__ int32_t wt[NWMAX][RN_THREADS / 64];
+    __shared__ uint32_t tau_hi[MF_MAXW];
+    // per width and wave: the largest box sum and its first position (only that wave writes them)
+    __shared__ double wv[MF_MAXW][RN_THREADS / 64];
+    __shared__ int32_t wt[MF_MAXW][RN_THREADS / 64];
     const int64_t b = blockIdx.x;
     const int64_t logical = (b % 8) * (gridDim.x / 8) + b / 8;
     if (logical >= nblocks) return;
@@ -599,9 +609,9 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
     const int64_t chunk = logical % nb_row;
     const NbRow r = rows[row];
     const int64_t n = r.n;
-    const int64_t t0 = chunk * RN_CHB;
+    const int64_t t0 = chunk * chb;
     if (t0 >= n || r.odd) return;
-    const int64_t tend = min<int64_t>(t0 + RN_CHB, n);  // the chunk's outputs
+    const int64_t tend = min<int64_t>(t0 + chb, n);  // the chunk's outputs
     const int64_t tn = min<int64_t>(tend + RN_SEG, n);  // samples normalised (one segment more)
     const int64_t wrapn = r.ng - n;                      // zt[n, Ng) = z[0, Ng - n)
     const int tid = threadIdx.x;
@@ -705,7 +715,8 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
         window_sums(0, H1, H2);
         norm_seg(0, nhead, h0, hn, hx, H1, H2, hz);
 #pragma unroll
-        for (int j = 0; j < RN_PER; ++j) head[RN_PER * tid + j] = hz[j];
+        for (int j = 0; j < RN_PER; ++j)
+            if (RN_PER * tid < nmirror) head[RN_PER * tid + j] = hz[j];
     }
 
     float c0[RN_PER], cn[RN_PER], cx[RN_PER];
@@ -713,28 +724,16 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
     double S1, S2;
     window_sums(t0, S1, S2);
     const int lane = tid & 63, wave = tid >> 6;
-    if (tid < NWMAX) tau_hi[tid] = 0;  // below every key; first read after the scans' barriers
-    double bestv[NWMAX];
-    int32_t bestt[NWMAX];  // position codes (segment << 3) | i
+    if (tid < MF_MAXW) {  // first read after the scans' barriers
+        tau_hi[tid] = 0;  // below every key
 #pragma unroll
-    for (int wi = 0; wi < NWMAX; ++wi) {
-        bestv[wi] = -INFINITY;
-        bestt[wi] = NB_NONE;
+        for (int k = 0; k < RN_THREADS / 64; ++k) {
+            wv[tid][k] = -INFINITY;
+            wt[tid][k] = NB_NOPOS;
+        }
     }
-    // The widths (<= MF_WMAX < 2^11), three to a VGPR: held in vector registers for the whole
-    // block (as scalars the compiler reloads them in the loop, and each reload's wait also
-    // drains the LDS reads in flight).
-    constexpr int NPACK = (NWMAX + 2) / 3;
-    uint32_t wpack[NPACK];
-#pragma unroll
-    for (int p = 0; p < NPACK; ++p) {
-        uint32_t v = 0;
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            if (3 * p + j < NWMAX && 3 * p + j < nw) v |= static_cast<uint32_t>(widths[3 * p + j]) << (11 * j);
-        asm volatile("v_mov_b32 %0, %1" : "=v"(wpack[p]) : "s"(v));
-    }
-    auto width_of = [&](int wi) { return static_cast<int>((wpack[wi / 3] >> (11 * (wi % 3))) & 0x7ffu); };
+    const int my_width = lane < nw ? widths[lane] : 0;
+    auto width_of = [&](int wi) { return __builtin_amdgcn_readlane(my_width, wi); };
     double carry = 0.0;  // P at the current segment's start
     double s_acc = 0.0;  // the thread's share of the chunk's z sum
     const int nseg = static_cast<int>((tend - t0 + RN_SEG - 1) / RN_SEG);
@@ -755,7 +754,7 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
                 const int64_t t = u0 + RN_PER * tid + j;
                 if (t >= n) {
                     const int64_t i = (t < r.ng) ? t - n : t - r.ng;
-                    z[j] = (i < nhead) ? head[i] : 0.f;
+                    z[j] = (i < min<int64_t>(nhead, nmirror)) ? head[i] : 0.f;  // no box reaches past them
                 }
             }
         }
@@ -780,13 +779,13 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
         double ex = tot, T;
         block_exscan1_total(ex, T, sa);
         {
-            // slots [0, MF_WMAX) are mirrored past the ring's end, so that a box of the
+            // slots [0, nmirror) are mirrored past the ring's end, so that a box of the
             // second half reads its far end without wrapping the index
             const int base = (k * RN_SEG + RN_PER * tid) & (NB_RING - 1);
             const double p0 = carry + ex;
 #pragma unroll
             for (int j = 0; j < RN_PER; ++j) ring[base + j] = p0 + pre[j];
-            if (base < MF_WMAX) {
+            if (base < nmirror) {
 #pragma unroll
                 for (int j = 0; j < RN_PER; ++j) ring[NB_RING + base + j] = p0 + pre[j];
             }
@@ -802,8 +801,6 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
             double q0[RN_PER];
 #pragma unroll
             for (int i = 0; i < RN_PER; ++i) q0[i] = rb[RN_THREADS * i];
-            // a thread's outputs are coded (segment << 3) | i, relative to this segment here
-            const int frame = (k - 1) << 3;
             // outputs past the chunk's end (last segment only) take no part
             int nvalid = RN_PER;
             if (!full) {
@@ -822,67 +819,60 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
                     }
                     return fmax(fmax(fmax(d[0], d[1]), fmax(d[2], d[3])), fmax(fmax(d[4], d[5]), fmax(d[6], d[7])));
                 };
+                const uint32_t my_tau = lane < nw ? tau_hi[lane] : 0u;
                 auto reaches = [&](int wi, double m) {
-                    return __any(static_cast<uint32_t>(order_key(m) >> 32) >= tau_hi[wi]) ? 1u : 0u;
+                    const uint32_t tau = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(my_tau), wi));
+                    return __any(static_cast<uint32_t>(order_key(m) >> 32) >= tau) ? 1u : 0u;
                 };
+                // the reads of the next width are in flight while one is reduced
                 uint32_t gate = 0;
-                if constexpr (EXACT) {
-                    // software-pipelined by hand: the reads of width wi + 1 are in flight while
-                    // width wi is reduced (the scheduling barriers keep the compiler from
-                    // hoisting every width's reads at once and spilling them)
-                    double buf[2][RN_PER];
-#pragma unroll
-                    for (int i = 0; i < RN_PER; ++i) buf[0][i] = rb[width_of(0) + RN_THREADS * i];
-#pragma unroll
-                    for (int wi = 0; wi < NWMAX; ++wi) {
-                        if (wi + 1 < NWMAX) {
-                            const double* __restrict__ rn = rb + width_of(wi + 1);
-#pragma unroll
-                            for (int i = 0; i < RN_PER; ++i) buf[(wi + 1) & 1][i] = rn[RN_THREADS * i];
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                        gate |= reaches(wi, max_of(buf[wi & 1])) << wi;
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                } else {
-#pragma unroll
-                    for (int wi = 0; wi < NWMAX; ++wi) {
-                        if (wi >= nw) continue;  // uniform
-                        const double* __restrict__ rw = rb + width_of(wi);
-                        double v[RN_PER];
-#pragma unroll
-                        for (int i = 0; i < RN_PER; ++i) v[i] = rw[RN_THREADS * i];
-                        gate |= reaches(wi, max_of(v)) << wi;
-                    }
-                }
-                // pass 2: exact first-maximum tracking per lane, for the widths whose bit is
-                // set. A lane whose sums stay below the block's largest tracked sum cannot hold
-                // the block's first maximum (every earlier position holds less than it);
-                // reaching it (>=) covers a tie with another wave's later position in this
-                // same segment. The test runs on the upper half of the order key, which can
-                // only let more lanes through.
-#pragma unroll
-                for (int wi = 0; wi < NWMAX; ++wi) {
-                    if (!((gate >> wi) & 1u)) continue;  // uniform
+                double even[RN_PER], odd[RN_PER];
+                auto read = [&](int wi, double (&v)[RN_PER]) {
                     const double* __restrict__ rw = rb + width_of(wi);
-                    const double old = bestv[wi];
-                    double bv = old;
-                    int32_t bc = bestt[wi] - frame;
+#pragma unroll
+                    for (int i = 0; i < RN_PER; ++i) v[i] = rw[RN_THREADS * i];
+                };
+                read(0, even);
+#pragma unroll 1
+                for (int wi = 0; wi < nw; wi += 2) {
+                    read(min(wi + 1, nw - 1), odd);
+                    __builtin_amdgcn_sched_barrier(0);
+                    gate |= reaches(wi, max_of(even)) << wi;
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (wi + 1 >= nw) break;
+                    read(min(wi + 2, nw - 1), even);
+                    __builtin_amdgcn_sched_barrier(0);
+                    gate |= reaches(wi + 1, max_of(odd)) << (wi + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // pass 2: the wave's first maximum of this segment, for the widths whose bit is
+                // set. A wave whose sums stay below the block's largest tracked sum cannot hold
+                // the block's first maximum (every earlier position holds less than it); reaching
+                // it (>=) covers a tie with another wave's later position in this same segment.
+                // The test runs on the upper half of the order key, which can only let more
+                // waves through.
+                while (gate) {
+                    const int wi = __builtin_ctz(gate);
+                    gate &= gate - 1;
+                    double v[RN_PER];
+                    read(wi, v);
+                    double bv = -INFINITY;
+                    int32_t bt = NB_NOPOS;
 #pragma unroll
                     for (int i = 0; i < RN_PER; ++i) {
-                        double di = rw[RN_THREADS * i] - q0[i];
+                        double di = v[i] - q0[i];
                         if constexpr (!decltype(all_valid)::value) di = (i < nvalid) ? di : -INFINITY;
                         const bool c = di > bv;  // strict: a tie keeps the lane's earlier position
                         bv = c ? di : bv;
-                        bc = c ? i : bc;
-                        // keeps each position select next to its compare (otherwise the compiler
-                        // hoists all compares and parks their masks in spilled registers)
-                        asm volatile("" : "+v"(bv), "+v"(bc));
+                        bt = c ? static_cast<int32_t>(a) + tid + RN_THREADS * i : bt;
                     }
-                    const uint32_t wk = wave_max_u32(static_cast<uint32_t>(order_key(bv) >> 32));
-                    if (lane == 0) atomicMax(&tau_hi[wi], wk);
-                    bestv[wi] = bv;
-                    bestt[wi] = bc + frame;
+                    const double m = wave_max(bv);
+                    const int32_t t = wave_min(bv == m ? bt : NB_NOPOS);
+                    if (lane == 0 && m > wv[wi][wave]) {  // strict: a tie keeps the earlier segment's
+                        wv[wi][wave] = m;
+                        wt[wi][wave] = t;
+                        atomicMax(&tau_hi[wi], static_cast<uint32_t>(order_key(m) >> 32));
+                    }
                 }
             };
             if (full)
@@ -892,20 +882,6 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
         }
     }
     // the block's first maximum per width: larger sum, then smaller position
-#pragma unroll
-    for (int wi = 0; wi < NWMAX; ++wi) {
-        if (wi >= nw) continue;  // uniform
-        const int32_t c = bestt[wi];
-        const int32_t t = (c == NB_NONE) ? NB_NOPOS
-                                         : static_cast<int32_t>(t0 + static_cast<int64_t>(c >> 3) * RN_SEG + tid +
-                                                                RN_THREADS * (c & 7));
-        const double v = wave_max(bestv[wi]);
-        const int32_t tw = wave_min(bestv[wi] == v ? t : NB_NOPOS);
-        if (lane == 0) {
-            wv[wi][wave] = v;
-            wt[wi][wave] = tw;
-        }
-    }
     const double s_blk = block_sum(s_acc, red);  // its barriers also order wv/wt
     if (tid < nw) {
         double v = wv[tid][0];
@@ -926,39 +902,41 @@ __global__ __launch_bounds__(RN_THREADS, NWMAX > 12 ? 2 : 3) void k_norm_boxcar(
 
 // Per row (one 64-thread block): S from the chunk sums in chunk order; per width (one thread
 // each) the first maximum over the chunks and conv_w; then the template-major first maximum.
-__global__ __launch_bounds__(64) void k_nb_final(const NbRow* __restrict__ rows, int64_t nb_row,
+__global__ __launch_bounds__(64) void k_nb_final(const NbRow* __restrict__ rows, int64_t nb_row, int64_t chb,
                                                  const int32_t* __restrict__ widths, int nw,
                                                  const double* __restrict__ part_s,
                                                  const double* __restrict__ part_v,
                                                  const int32_t* __restrict__ part_t, float* __restrict__ snr,
                                                  int32_t* __restrict__ peak, int32_t* __restrict__ widx) {
-    __shared__ double S_sh;
     __shared__ float cv_sh[MF_MAXW];
     __shared__ int32_t t_sh[MF_MAXW];
     const int64_t row = blockIdx.x;
     const NbRow r = rows[row];
     if (r.odd) return;  // the FFT path writes this row's result
-    const int64_t nch = (r.n + RN_CHB - 1) / RN_CHB;
+    const int64_t nch = (r.n + chb - 1) / chb;
     const int lane = threadIdx.x;
-    if (lane == 0) {
-        double S = 0.0;
-        for (int64_t c = 0; c < nch; ++c) S += part_s[row * nb_row + c];
-        S_sh = S;
+    // S: the chunk sums loaded 64 at a time, added in chunk order
+    double S = 0.0;
+    for (int64_t c0 = 0; c0 < nch; c0 += 64) {
+        const double v = c0 + lane < nch ? part_s[row * nb_row + c0 + lane] : 0.0;
+        const int m = static_cast<int>(min<int64_t>(64, nch - c0));
+        for (int k = 0; k < m; ++k) S += __shfl(v, k);
     }
-    __syncthreads();
     if (lane < nw) {
         double bv = -INFINITY;
         int32_t bt = NB_NOPOS;
+#pragma unroll 8
         for (int64_t c = 0; c < nch; ++c) {
             const int64_t i = (row * nb_row + c) * MF_MAXW + lane;
             const double v = part_v[i];
+            const int32_t t = part_t[i];
             if (v > bv) {  // chunks in time order: a tie keeps the earlier one
                 bv = v;
-                bt = part_t[i];
+                bt = t;
             }
         }
         const double w = widths[lane], ng = static_cast<double>(r.ng);
-        cv_sh[lane] = static_cast<float>((bv - w * S_sh / ng) * (1.0 / sqrt(w * (1.0 - w / ng))));
+        cv_sh[lane] = static_cast<float>((bv - w * S / ng) * (1.0 / sqrt(w * (1.0 - w / ng))));
         t_sh[lane] = bt;
     }
     __syncthreads();
@@ -1264,12 +1242,24 @@ namespace {
 // k_norm_boxcar; for rows with an odd good size one row's z, taps, convs, FFT space and
 // chunk partials, reused row after row.
 struct NbLayout {
-    int64_t nb_row = 0, off_rows = 0, off_w = 0, off_s = 0, off_v = 0, off_t = 0;
+    int64_t chb = 0, nb_row = 0, off_rows = 0, off_w = 0, off_s = 0, off_v = 0, off_t = 0;
     int64_t odd_n = 0, nodd = 0, fft_bytes = 0;
     int64_t off_rd = 0, off_mrow = 0, off_z = 0, off_td = 0, off_taps = 0, off_convs = 0, off_fft = 0,
             off_part = 0;
     int64_t bytes = 0;
 };
+
+// Outputs per block: 16 segments (one more is normalised for the boxes past a block's end, and
+// its first window summed), or fewer while that leaves most of 256 CUs' four block slots empty.
+// 301 x 160007 samples, 14 widths: 372 us with 16 segments (1505 blocks), 393 with 8, 443 with 4;
+// 64 x 65536, 9 widths: 149 with 16 (128 blocks), 121 with 8, 114 with 4; one row of 262144, 14
+// widths: 155 with 16, 108 with 2 (times of whole calls, about 90 us of them not in the kernel).
+int64_t nb_chunk(int64_t nrows, int64_t max_len) {
+    int64_t segs = 16;
+    while (segs > 2 && nrows * spp::ceil_div(max_len, segs * RN_SEG) < 512) segs /= 2;
+    return segs * RN_SEG;
+}
+
 NbLayout nb_layout(int64_t nrows, const int64_t* row_len, const int32_t* widths, int32_t nw) {
     NbLayout l;
     int64_t max_len = 1, sumw = 0;
@@ -1283,7 +1273,8 @@ NbLayout nb_layout(int64_t nrows, const int64_t* row_len, const int32_t* widths,
         }
     }
     for (int i = 0; i < nw; ++i) sumw += widths[i];
-    l.nb_row = std::max<int64_t>(1, spp::ceil_div(max_len, RN_CHB));
+    l.chb = nb_chunk(nrows, max_len);
+    l.nb_row = std::max<int64_t>(1, spp::ceil_div(max_len, l.chb));
     int64_t off = 0;
     l.off_rows = off; off = align256(off + static_cast<int64_t>(sizeof(NbRow)) * nrows);
     l.off_w = off; off = align256(off + 4 * MF_MAXW);
@@ -1304,17 +1295,6 @@ NbLayout nb_layout(int64_t nrows, const int64_t* row_len, const int32_t* widths,
     return l;
 }
 
-template <int NWMAX, bool EXACT>
-void launch_norm_boxcar(bool aligned, dim3 grid, hipStream_t st, const float* x, int64_t ldx, const NbRow* rows,
-                        int64_t nb_row, int64_t nblocks, int32_t window, const int32_t* widths, int nw,
-                        int32_t wmax, double* ps, double* pv, int32_t* pt) {
-    if (aligned)
-        hipLaunchKernelGGL((k_norm_boxcar<NWMAX, EXACT, true>), grid, dim3(RN_THREADS), 0, st, x, ldx, rows, nb_row,
-                           nblocks, window, widths, nw, wmax, ps, pv, pt);
-    else
-        hipLaunchKernelGGL((k_norm_boxcar<NWMAX, EXACT, false>), grid, dim3(RN_THREADS), 0, st, x, ldx, rows,
-                           nb_row, nblocks, window, widths, nw, wmax, ps, pv, pt);
-}
 }  // namespace
 
 extern "C" int spp_normalise_boxcar_mf_workspace_size(int64_t nrows, const int64_t* row_len_host,
@@ -1389,19 +1369,15 @@ extern "C" int spp_normalise_boxcar_mf(const float* x, int64_t ldx, int64_t nrow
     const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && ldx % 4 == 0 && L % 4 == 0 &&
                          (window - L) % 4 == 0;
     const dim3 grid(static_cast<unsigned>(spp::ceil_div(nblocks, int64_t(8)) * 8));
-    // the width loops are unrolled: exactly 9 widths (the doubling ladder 1..256), up to 12,
-    // up to 32
-    if (nwidths == 9)
-        launch_norm_boxcar<9, true>(aligned, grid, st, x, ldx, drows, l.nb_row, nblocks, window, dw, nwidths, wmax,
-                                    ps, pv, pt);
-    else if (nwidths <= 12)
-        launch_norm_boxcar<12, false>(aligned, grid, st, x, ldx, drows, l.nb_row, nblocks, window, dw, nwidths, wmax,
-                                      ps, pv, pt);
+    const auto lds = static_cast<unsigned>(nb_lds_bytes(wmax));
+    if (aligned)
+        hipLaunchKernelGGL((k_norm_boxcar<true>), grid, dim3(RN_THREADS), lds, st, x, ldx, drows, l.nb_row, l.chb,
+                           nblocks, window, dw, nwidths, wmax, ps, pv, pt);
     else
-        launch_norm_boxcar<MF_MAXW, false>(aligned, grid, st, x, ldx, drows, l.nb_row, nblocks, window, dw, nwidths,
-                                           wmax, ps, pv, pt);
+        hipLaunchKernelGGL((k_norm_boxcar<false>), grid, dim3(RN_THREADS), lds, st, x, ldx, drows, l.nb_row, l.chb,
+                           nblocks, window, dw, nwidths, wmax, ps, pv, pt);
     SPP_LAUNCHED("k_norm_boxcar");
-    hipLaunchKernelGGL(k_nb_final, dim3(static_cast<unsigned>(nrows)), dim3(64), 0, st, drows, l.nb_row, dw,
+    hipLaunchKernelGGL(k_nb_final, dim3(static_cast<unsigned>(nrows)), dim3(64), 0, st, drows, l.nb_row, l.chb, dw,
                        nwidths, ps, pv, pt, snr, peak, widx);
     SPP_LAUNCHED("k_nb_final");
     // Rows with an odd good size, one after the other: z through k_norm, the template bank

@@ -131,3 +131,15 @@ def test_sweep_result_matched_filter_uses_one_pass():
     plane = plan.execute(_lib.to_device(data.reshape(-1)))
     res = SweepResult(plane, plan.row_len, np.arange(3.0), header=None, plan=plan, table=table)
     _compare(res.matched_filter(4096, W9), _two_pass(plane, plan.row_len, 4096, W9), "sweep rows")
+
+
+@pytest.mark.parametrize("nwidths", [1, 2, 13, 31, 32])
+@pytest.mark.parametrize("nrows", [1, 40])
+def test_fused_block_lengths_and_width_counts(nrows, nwidths):
+    """Few rows take shorter blocks (2 to 16 segments); any number of widths is one kernel."""
+    rng = np.random.default_rng(100 * nrows + nwidths)
+    widths = sorted(rng.choice(np.arange(1, 513), nwidths, replace=False).tolist())
+    n = 5 * 2048 + 17 if nrows == 1 else 16 * 2048 * 3 - 1
+    row_len = [n - 3 * i for i in range(nrows)]
+    x = _rows(rng, row_len, n + 5, integer=True, pulses=[(0, 4090, widths[-1], 300.0), (nrows - 1, n - 5, 9, 500.0)])
+    _compare(_fused(x, row_len, 4096, widths), _two_pass(x, row_len, 4096, widths), f"{nrows} rows")
