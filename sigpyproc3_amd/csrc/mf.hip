@@ -963,14 +963,36 @@ __global__ __launch_bounds__(64) void k_nb_final(const NbRow* __restrict__ rows,
 
 using spp::TempDesc;
 
+// Partial sums of zt over [0, Ng), CT_PARTS of them; every convolution wave adds them in one
+// fixed order. (One block summing 262144 samples took 136 us.)
+constexpr int CT_PARTS = 64;
+__global__ __launch_bounds__(MF_THREADS) void k_circ_parts(const float* __restrict__ z, int64_t n, int64_t ng,
+                                                           double* __restrict__ parts) {
+    __shared__ double red[MF_THREADS / 64];
+    const int64_t per = (ng + CT_PARTS - 1) / CT_PARTS;
+    const int64_t i0 = static_cast<int64_t>(blockIdx.x) * per, i1 = min(i0 + per, ng);
+    double s = 0.0;
+#pragma unroll 4
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += MF_THREADS) s += static_cast<double>(z[i >= n ? i - n : i]);  // ng < 2n
+    s = block_sum(s, red);
+    if (threadIdx.x == 0) parts[blockIdx.x] = s;
+}
+
+// One block per CT_B outputs and template, CT_R consecutive outputs per thread: four taps and four
+// new samples come from two LDS reads each and feed 16 float64 multiply-adds (with one output at a
+// time every multiply-add read both its factors from LDS). Each output adds its taps in order.
+// 262144 samples, 13 gaussians of up to 381 taps: 53 -> 30 us (FP64 issue: 3e8 multiply-adds, and a conversion per LDS value).
+constexpr int CT_R = 4;
+static_assert(CT_R * MF_THREADS == CT_B, "every thread has CT_R outputs");
 __global__ __launch_bounds__(MF_THREADS) void k_template_conv(
-    const float* __restrict__ z, int64_t n, int64_t ng, const double* __restrict__ S,
+    const float* __restrict__ z, int64_t n, int64_t ng, const double* __restrict__ parts,
     const float* __restrict__ taps, const TempDesc* __restrict__ temps, float* __restrict__ convs) {
-    __shared__ float zs[CT_B + CT_TAPS];
-    __shared__ float hs[CT_TAPS];
+    __shared__ __align__(16) float zs[CT_B + CT_TAPS];
+    __shared__ __align__(16) double hs[CT_TAPS];
     const int64_t a = static_cast<int64_t>(blockIdx.x) * CT_B;
     const TempDesc td = temps[blockIdx.y];
     const int tid = threadIdx.x;
+    const double total = lane63(wave_incl_scan(parts[tid & 63]));
     // zt[(t - ref + m) mod Ng] for t in [a, a + CT_B), m < len.
     const int nel = CT_B + td.len - 1;
     for (int k = tid; k < nel; k += MF_THREADS) {
@@ -979,27 +1001,43 @@ __global__ __launch_bounds__(MF_THREADS) void k_template_conv(
         i = wrap_index(i, ng);
         zs[k] = z[wrap_index(i, n)];  // ng < 2n
     }
-    for (int m = tid; m < td.len; m += MF_THREADS) hs[m] = taps[td.off + m];
+    for (int m = tid; m < td.len; m += MF_THREADS) hs[m] = static_cast<double>(taps[td.off + m]);
     __syncthreads();
     double mu, inv;
     spp::temp_norm(td, ng, &mu, &inv);
-    const double mus = mu * S[0];
-    for (int u = tid; u < CT_B; u += MF_THREADS) {
-        const int64_t t = a + u;
-        if (t >= n) break;
-        double acc = 0.0;
-        for (int m = 0; m < td.len; ++m) acc += static_cast<double>(hs[m]) * static_cast<double>(zs[u + m]);
-        convs[static_cast<int64_t>(blockIdx.y) * n + t] = static_cast<float>((acc - mus) * inv);
+    const double mus = mu * total;
+    const int u = CT_R * tid;
+    const int64_t t = a + u;
+    if (t >= n) return;
+    double acc[CT_R] = {};
+    double x[2 * CT_R];  // zt at the outputs' positions for taps m .. m + CT_R - 1
+    auto load4 = [&](int k, double* __restrict__ d) {
+        const float4 v = *reinterpret_cast<const float4*>(&zs[u + k]);
+        d[0] = v.x;
+        d[1] = v.y;
+        d[2] = v.z;
+        d[3] = v.w;
+    };
+    load4(0, x);
+    int m = 0;
+    for (; m + CT_R <= td.len; m += CT_R) {
+        load4(m + CT_R, x + CT_R);
+        const double2 h01 = *reinterpret_cast<const double2*>(&hs[m]);
+        const double2 h23 = *reinterpret_cast<const double2*>(&hs[m + 2]);
+        const double h[CT_R] = {h01.x, h01.y, h23.x, h23.y};
+#pragma unroll
+        for (int k = 0; k < CT_R; ++k)
+#pragma unroll
+            for (int r = 0; r < CT_R; ++r) acc[r] += h[k] * x[r + k];
+#pragma unroll
+        for (int r = 0; r < CT_R; ++r) x[r] = x[r + CT_R];
     }
-}
-
-__global__ __launch_bounds__(MF_THREADS) void k_circ_sum1(const float* __restrict__ z, int64_t n,
-                                                          int64_t ng, double* __restrict__ S) {
-    __shared__ double red[MF_THREADS];
-    double s = 0.0;
-    for (int64_t i = threadIdx.x; i < ng; i += MF_THREADS) s += static_cast<double>(z[wrap_index(i, n)]);
-    s = block_sum(s, red);
-    if (threadIdx.x == 0) S[0] = s;
+    for (; m < td.len; ++m)
+#pragma unroll
+        for (int r = 0; r < CT_R; ++r) acc[r] += hs[m] * static_cast<double>(zs[u + r + m]);
+#pragma unroll
+    for (int r = 0; r < CT_R; ++r)
+        if (t + r < n) convs[static_cast<int64_t>(blockIdx.y) * n + t + r] = static_cast<float>((acc[r] - mus) * inv);
 }
 
 using spp::good_size_real;
@@ -1490,7 +1528,7 @@ struct CtLayout {
 };
 CtLayout ct_layout(int64_t n, int32_t ntemps, int64_t total_taps) {
     CtLayout l;
-    int64_t off = align256(8);
+    int64_t off = align256(8 * CT_PARTS);
     l.off_td = off; off = align256(off + static_cast<int64_t>(sizeof(TempDesc)) * ntemps);
     l.off_taps = off; off = align256(off + 4 * total_taps);
     const int64_t ng = good_size_real(n);
@@ -1561,8 +1599,8 @@ extern "C" int spp_convolve_templates(const float* data, int64_t n, const float*
         const int rc = spp::odd_convolve(data, n, taps, dtd, ntemps, convs, n, ws + l.off_fft, l.fft_bytes, st);
         if (rc != SPP_OK) return rc;
     } else {
-        hipLaunchKernelGGL(k_circ_sum1, dim3(1), dim3(MF_THREADS), 0, st, data, n, ng, S);
-        SPP_LAUNCHED("k_circ_sum1");
+        hipLaunchKernelGGL(k_circ_parts, dim3(CT_PARTS), dim3(MF_THREADS), 0, st, data, n, ng, S);
+        SPP_LAUNCHED("k_circ_parts");
         hipLaunchKernelGGL(k_template_conv,
                            dim3(static_cast<unsigned>(spp::ceil_div(n, CT_B)), static_cast<unsigned>(ntemps)),
                            dim3(MF_THREADS), 0, st, data, n, ng, S, taps, dtd, convs);
