@@ -68,7 +68,10 @@ constexpr int build_lds_bytes() {
 // builds words j0 + 4q .. 4q+3 of every channel packed in byte column bc from one LDS byte
 // per (row, word) and stores them as one 16-byte write per channel (a wave writes 512
 // contiguous bytes per channel). Only the first glen words of each channel row are written
-// (the sweep reads no further). One barrier, reached by every thread of the block. MAXB bounds
+// (the sweep reads no further). One barrier, reached by every thread of the block. ALIGNED: rows
+// are whole dwords on a 4-byte aligned stream; otherwise rows of at least 4 bytes are loaded by
+// dwords at any byte (1002 4-bit channels x 100003 samples: 178 us with a load per byte, 132 so),
+// and narrower ones (row_bytes < 4) by bytes. MAXB bounds
 // the staging loads in flight per thread (registers); tid is the thread's index in the block
 // of NT threads (B_THREADS or a multiple).
 template <int NBITS, bool BIG, bool ALIGNED, int BCW, int MAXB = 32, int NT = B_THREADS>
@@ -106,9 +109,17 @@ __device__ __forceinline__ void build_tile(const uint8_t* __restrict__ in, int64
                 if (ALIGNED) {
                     // row_bytes and the stream start are multiples of 4: whole dwords or none
                     if (left > 0) v[i] = *reinterpret_cast<const uint32_t*>(src);
+                } else if (row_bytes >= 4) {
+                    // a dword at any byte, moved back to end with the row where it would cross it
+                    if (left > 0) {
+                        const int back = left < 4 ? 4 - static_cast<int>(left) : 0;
+                        uint32_t d;
+                        __builtin_memcpy(&d, src - back, 4);
+                        v[i] = d >> (8 * back);
+                    }
                 } else {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
+                    for (int u = 0; u < 3; ++u)
                         if (u < left) v[i] |= static_cast<uint32_t>(src[u]) << (8 * u);
                 }
             }
