@@ -365,15 +365,16 @@ int fill_f32(float* p, int64_t n, hipStream_t st) {
     return SPP_OK;
 }
 
-// The dedisperse form with word-parallel adds (gulp_swar.hip), for rows of whole dwords.
+// The dedisperse form with word-parallel adds (gulp_swar.hip), for rows of at least four bytes.
 // Channels are grouped as below, with the SWAR kernel's stage (a fixed run of dwords of each
 // row) in place of DD_CC channels and its own time tile.
 int launch_swar(const uint8_t* in, int nbits, int big, const int32_t* delays, float* out, int64_t nchans,
                 int64_t nsamps, int64_t nout, int64_t out_start, hipStream_t st) {
     const int64_t row_bytes = nchans * nbits / 8;
-    const bool compact = spp::gulp_swar_compact(nbits, nchans, nsamps - nout);
+    const bool aligned = row_bytes % 4 == 0 && reinterpret_cast<uintptr_t>(in) % 4 == 0;
+    const spp::GulpForm form = spp::gulp_swar_form(nbits, aligned, nchans, nout, nsamps - nout);
     const int64_t T = spp::gulp_swar_tile(nbits);
-    const int64_t chunk = spp::gulp_swar_stage_channels(nbits);  // channels of one stage
+    const int64_t chunk = spp::gulp_swar_stage_channels(nbits, form);  // channels of one stage
     const int64_t bx = spp::ceil_div(nout, T);
     SPP_REQUIRE(bx <= 0x7fffffffLL, "gulp too long");
     const int64_t cus = spp::device_cu_count();
@@ -388,7 +389,10 @@ int launch_swar(const uint8_t* in, int nbits, int big, const int32_t* delays, fl
     int64_t ilv = 1, nchunk = 1;
     const int64_t line_ch = 1024 / nbits;  // channels in a 128-byte row line
     const int64_t line_spread = (nsamps - nout) * line_ch / nchans;
-    const bool wide_groups = exact && cpg >= chunk && nchans >= line_ch && nchans % line_ch == 0;
+    // Also for rows that are not whole lines (neighbouring chunks still share most lines): 8-bit 1000
+    // channels x 200000 samples 200 us in contiguous groups, 86 with the line's groups side by side;
+    // not for 4-bit ones (1000 x 200000: 62 / 68).
+    const bool wide_groups = exact && cpg >= chunk && nchans >= line_ch && (nbits != 4 || nchans % line_ch == 0);
     if (wide_groups && line_spread <= T) {
         cpg = chunk;
         ilv = line_ch / chunk;
@@ -407,14 +411,14 @@ int launch_swar(const uint8_t* in, int nbits, int big, const int32_t* delays, fl
         if (rc) return rc;
     }
     return spp::launch_gulp_swar(in, nbits, big != 0, delays, out, nchans, nsamps, nout, out_start, row_bytes, cpg,
-                                 groups, ilv, nchunk, use_atomic, compact, st);
+                                 groups, ilv, nchunk, use_atomic, form, st);
 }
 
 template <int MODE>
 int launch_int(const uint8_t* in, int nbits, int big, const int32_t* delays, const int32_t* cts,
                float* out, int64_t nchans, int64_t nsamps, int64_t nout, int64_t out_start,
                int64_t nsubs, int64_t out_size, hipStream_t st) {
-    if (MODE == 0 && spp::gulp_swar_applies(in, nbits, nchans))
+    if (MODE == 0 && spp::gulp_swar_applies(nbits, nchans))
         return launch_swar(in, nbits, big, delays, out, nchans, nsamps, nout, out_start, st);
     const int64_t row_bytes = nchans * nbits / 8;
     const int64_t bx = spp::ceil_div(nout, DD_T);

@@ -1,8 +1,8 @@
 // One-DM dedispersion of a packed 1/2/4/8-bit gulp with word-parallel adds: the dedisperse
-// form of kernels.dedisperse (core/kernels.py:340-362) for integer samples, when every
-// packed row is whole dwords.
+// form of kernels.dedisperse (core/kernels.py:340-362) for integer samples in rows of at
+// least four bytes.
 //
-// A block owns T consecutive outputs and a group of channels, taken in stages of GS_S packed
+// A block owns T consecutive outputs and a group of channels, taken in stages of S packed
 // dword columns (16 bytes of each row; F = 32/nbits channels per dword). Staging turns rows
 // into channel-major series: a thread loads F consecutive rows of one dword column (an F x F
 // block of samples), transposes it in registers by delta swaps (log2 F rounds of shift,
@@ -30,10 +30,7 @@
 
 namespace {
 
-constexpr int GS_THREADS = 256;
-constexpr int GS_S = 4;     // dword columns per stage (16 bytes of each row)
-constexpr int GS_LOGS = 2;  // log2(GS_S)
-constexpr int GS_RMAX = 2560;  // rows one pass stages at most (the compact form: fewer, below)
+constexpr int GS_SMAX = 8;  // dword columns per stage at most
 // Word 3 of a raw buffer resource on gfx9-family GPUs: 32-bit data format, no swizzle.
 constexpr int kBufferFlags = 0x00020000;
 
@@ -45,23 +42,36 @@ constexpr int series_pitch(int f, int nrb) {
     return nrb + 1;
 }
 
-// COMPACT (4/8-bit data): a series buffer of half the rows, about 21 KB, so that twice as many
-// blocks share a CU (these kernels are bound by LDS size, not registers) when the stages' delay
-// spreads are small. 1/2-bit blocks are register-bound: more LDS room buys them nothing.
-template <int NBITS, bool COMPACT = false>
+// Block forms. NORMAL: 256 threads, stages of 16 bytes of each row. COMPACT (4/8-bit data): a series
+// buffer of half the rows, about 21 KB, so that twice as many blocks share a CU (these kernels
+// are bound by LDS size, not registers) when the stages' delay spreads are small; 1/2-bit
+// blocks are register-bound: more LDS room buys them nothing. WIDE (2-bit data; 8-bit data with
+// the compact buffer): 512 threads and 32 bytes of each row, so that half as many CUs refill a
+// row's line from L2, for long gulps whose wider stages still fit one pass. Measured, wide against
+// the narrow form: 2-bit 4096 channels x 2^20 at DM 557 475 / 582 us, x 2^18 at DM 0 110 / 135 but
+// at DM 1000 (two passes a stage) 149 / 131; 8-bit 3180 x 119779 at DM 300 152 / 205, 4096 x 2^18
+// 363 / 409, but 1024 x 65536 35 / 32.5. 1- and 4-bit data lose (1-bit 4096 x 2^18: 133 / 88).
+using spp::GulpForm;
+template <int NBITS, GulpForm FORM>
 struct Geo {
+    static constexpr bool WIDE = FORM == GulpForm::wide;
     static constexpr int F = 32 / NBITS;                                    // samples per dword
     static constexpr int T = (NBITS == 8 || NBITS == 4) ? 1024 : 2048;     // outputs per block
-    static constexpr int RMAX = COMPACT ? 1280 : GS_RMAX;
-    static constexpr int NG = T / F > GS_THREADS ? T / F / GS_THREADS : 1;  // output groups per thread
+    static constexpr int THREADS = WIDE ? 512 : 256;
+    static constexpr int S = WIDE ? 8 : 4;  // dword columns per stage
+    static constexpr int LOGS = WIDE ? 3 : 2;
+    // rows one pass stages at most
+    static constexpr int RMAX = FORM == GulpForm::compact || (WIDE && NBITS == 8) ? 1280 : (WIDE ? 2432 : 2560);
+    static constexpr int NG = T / F > THREADS ? T / F / THREADS : 1;  // output groups per thread
     static constexpr int G = T / F / NG;                                    // threads per partition
-    static constexpr int H = GS_THREADS / G;                                // channel partitions
+    static constexpr int H = THREADS / G;                                   // channel partitions
     static constexpr int NRB = RMAX / F;                                    // series dwords used
     static constexpr int PITCH = series_pitch(F, NRB);
     static constexpr int SPREAD = RMAX - T - 2 * F;                         // per pass
-    static constexpr int CH = GS_S * F;                                     // channels per stage
-    static_assert(G * H == GS_THREADS && G >= 64 && G * NG * F == T, "a wave's lanes share one channel partition");
-    static_assert(!COMPACT || NBITS >= 4, "compact form for byte-wide and nibble-wide samples only");
+    static constexpr int CH = S * F;                                        // channels per stage
+    static_assert(G * H == THREADS && G >= 64 && G * NG * F == T, "a wave's lanes share one channel partition");
+    static_assert(FORM != GulpForm::compact || NBITS >= 4, "compact form for byte-wide and nibble-wide samples only");
+    static_assert(!WIDE || NBITS == 2 || NBITS == 8, "wide form for 2- and 8-bit samples only");
 };
 
 constexpr uint32_t swap_mask(int s) {
@@ -244,18 +254,22 @@ struct SwarAcc<8> {  // 16-bit fields (257 channels), 32-bit
     }
 };
 
-template <int NBITS, bool BIG, bool COMPACT>
-__global__ __launch_bounds__(GS_THREADS, 3) void k_gulp_swar(
+// ALIGNED: rows are whole dwords on a 4-byte aligned stream. Otherwise the columns are loaded by
+// dwords at any byte; a row's last column, which its end may cut, is moved back to end with
+// the row and shifted, so that the channels it lacks read as 0.
+template <int NBITS, bool BIG, GulpForm FORM, bool ALIGNED>
+__global__ __launch_bounds__((Geo<NBITS, FORM>::THREADS), (FORM == GulpForm::wide ? 4 : 3)) void k_gulp_swar(
     const uint8_t* __restrict__ in, const int32_t* __restrict__ delays, float* __restrict__ out, int64_t nchans,
     int64_t nsamps, int64_t nout, int64_t out_start, int64_t row_bytes, int64_t chans_per_group, int64_t ngroups,
     int64_t nblocks, int64_t ilv, int64_t nchunk, int use_atomic) {
-    using Gm = Geo<NBITS, COMPACT>;
+    using Gm = Geo<NBITS, FORM>;
+    constexpr int S = Gm::S, LOGS = Gm::LOGS, THREADS = Gm::THREADS;
     constexpr int F = Gm::F, T = Gm::T, G = Gm::G, H = Gm::H, NG = Gm::NG, PITCH = Gm::PITCH, CH = Gm::CH;
     constexpr int UNITS = F >= 32 ? 1 : 2;  // staging units in flight per thread
     __shared__ uint32_t series[CH * PITCH];
     __shared__ __align__(16) int32_t sdel[CH];
     __shared__ int2 cinfo[CH];  // per stage channel: series index of its first dword, funnel shift
-    __shared__ int32_t cmin[GS_S], cmax[GS_S];
+    __shared__ int32_t cmin[GS_SMAX], cmax[GS_SMAX];
     // XCD-aware order, as the byte-staged kernel: the groups of one time tile are consecutive
     // logical blocks on one XCD, and share the packed row lines in its L2.
     const int64_t per_xcd = gridDim.x / 8;
@@ -276,7 +290,7 @@ __global__ __launch_bounds__(GS_THREADS, 3) void k_gulp_swar(
         c = cb + j * CH;
         const int64_t ce = min(nchans, cb + chans_per_group);
         if (c >= ce) return false;  // past nchans: so are all later chunks
-        nch = static_cast<int>(min<int64_t>(CH, ce - c));  // a multiple of F
+        nch = static_cast<int>(min<int64_t>(CH, (ce - c + F - 1) / F * F));  // whole columns
         return true;
     };
     const int64_t spc = (chans_per_group + CH - 1) / CH;  // stages per chunk
@@ -302,12 +316,33 @@ __global__ __launch_bounds__(GS_THREADS, 3) void k_gulp_swar(
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint8_t*>(in) + (inside ? rbase * row_bytes + col0 : 0), 0,
             inside ? static_cast<int>(span) : 0, kBufferFlags);
-        // unit u -> (column u % nqp, row block u / nqp); shifts when the pass has all GS_S columns
-        const bool full_width = nqp == GS_S;
-        auto unit_col = [&](int u) { return full_width ? (u & (GS_S - 1)) : u % nqp; };
-        auto unit_blk = [&](int u) { return full_width ? (u >> GS_LOGS) : u / nqp; };
+        // unit u -> (column u % nqp, row block u / nqp); shifts when the pass has all S columns
+        const bool full_width = nqp == S;
+        auto unit_col = [&](int u) { return full_width ? (u & (S - 1)) : u % nqp; };
+        auto unit_blk = [&](int u) { return full_width ? (u >> LOGS) : u / nqp; };
         auto load_unit = [&](int u, uint32_t (&w)[F]) {
             const int qq = unit_col(u), b = unit_blk(u);
+            if constexpr (!ALIGNED) {
+                const int64_t col = col0 + 4 * qq;
+                const int back = static_cast<int>(max<int64_t>(0, col + 4 - row_bytes));
+                const int64_t r0 = rbase + int64_t(F) * b;
+                if (inside) {
+                    const uint8_t* p = in + r0 * row_bytes + col - back;
+#pragma unroll
+                    for (int k = 0; k < F; ++k) __builtin_memcpy(&w[k], p + k * row_bytes, 4);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < F; ++k) {
+                        int64_t row = r0 + k;
+                        if (row < 0) row += nsamps;  // numba wraparound of a negative index
+                        w[k] = 0;
+                        if (row >= 0 && row < nsamps) __builtin_memcpy(&w[k], in + row * row_bytes + col - back, 4);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < F; ++k) w[k] >>= 8 * back;
+                return;
+            }
             if (inside) {
                 const uint32_t off = static_cast<uint32_t>(F * b) * static_cast<uint32_t>(row_bytes) + 4u * qq;
 #pragma unroll
@@ -333,14 +368,14 @@ __global__ __launch_bounds__(GS_THREADS, 3) void k_gulp_swar(
 #pragma unroll
             for (int p = 0; p < F; ++p) series[(cq + chan_of<NBITS, BIG>(p)) * PITCH + b] = w[p];
         };
-        for (int u = tid; u < units; u += UNITS * GS_THREADS) {
+        for (int u = tid; u < units; u += UNITS * THREADS) {
             uint32_t w[UNITS][F];
 #pragma unroll
             for (int i = 0; i < UNITS; ++i)
-                if (u + i * GS_THREADS < units) load_unit(u + i * GS_THREADS, w[i]);
+                if (u + i * THREADS < units) load_unit(u + i * THREADS, w[i]);
 #pragma unroll
             for (int i = 0; i < UNITS; ++i)
-                if (u + i * GS_THREADS < units) store_unit(u + i * GS_THREADS, w[i]);
+                if (u + i * THREADS < units) store_unit(u + i * THREADS, w[i]);
         }
         __syncthreads();
         // Summing: this thread's outputs t0 + F (g + G i) + j over its share of the pass's
@@ -379,7 +414,8 @@ __global__ __launch_bounds__(GS_THREADS, 3) void k_gulp_swar(
     int64_t c = 0, sm = 0, sj = 0;
     int nch = 0;
     bool have = stage_at(0, 0, c, nch);
-    int32_t dpre = (have && tid < nch) ? delays[c + tid] : 0;
+    // a cut column's missing channels (all 0) go with the last channel's delay
+    int32_t dpre = (have && tid < nch) ? delays[min<int64_t>(c + tid, nchans - 1)] : 0;
     while (have) {
         __syncthreads();  // the previous stage's tables and series are no longer read
         if (tid < nch) sdel[tid] = dpre;
@@ -390,7 +426,7 @@ __global__ __launch_bounds__(GS_THREADS, 3) void k_gulp_swar(
         int64_t cn = 0;
         int nchn = 0;
         const bool haven = stage_at(sm, sj, cn, nchn);
-        if (haven && tid < nchn) dpre = delays[cn + tid];  // the next stage's delays load meanwhile
+        if (haven && tid < nchn) dpre = delays[min<int64_t>(cn + tid, nchans - 1)];  // the next stage's delays load meanwhile
         __syncthreads();
         const int nq = nch / F;
         if (tid < nq) {
@@ -454,7 +490,7 @@ __global__ __launch_bounds__(GS_THREADS, 3) void k_gulp_swar(
     }
     __syncthreads();
     float* dst = out + out_start;
-    for (int t = tid; t < T; t += GS_THREADS) {
+    for (int t = tid; t < T; t += THREADS) {
         uint32_t s = 0;
 #pragma unroll
         for (int hh = 0; hh < H; ++hh) s += series[hh * T + t];
@@ -479,48 +515,65 @@ int64_t swar_max_channels(int nbits) {
 namespace spp {
 
 int64_t gulp_swar_tile(int nbits) {
-    return nbits == 8 ? Geo<8>::T : (nbits == 4 ? Geo<4>::T : (nbits == 2 ? Geo<2>::T : Geo<1>::T));
+    return nbits == 8 ? Geo<8, GulpForm::normal>::T
+                      : (nbits == 4 ? Geo<4, GulpForm::normal>::T
+                                    : (nbits == 2 ? Geo<2, GulpForm::normal>::T : Geo<1, GulpForm::normal>::T));
 }
 
-bool gulp_swar_compact(int nbits, int64_t nchans, int64_t max_delay) {
-    if (nbits < 4 || nchans <= 0) return false;
-    const int64_t spread = nbits == 8 ? Geo<8, true>::SPREAD : Geo<4, true>::SPREAD;
-    // twice the mean delay spread of a stage's channels (the widest stages of a dispersion
-    // sweep run 1.4-1.6 times the mean)
-    return 2 * max_delay * gulp_swar_stage_channels(nbits) <= spread * nchans;
+int64_t gulp_swar_stage_channels(int nbits, GulpForm form) {
+    return int64_t(form == GulpForm::wide ? Geo<2, GulpForm::wide>::S : Geo<2, GulpForm::normal>::S) * (32 / nbits);
 }
 
-int64_t gulp_swar_stage_channels(int nbits) { return int64_t(GS_S) * (32 / nbits); }
+GulpForm gulp_swar_form(int nbits, bool aligned, int64_t nchans, int64_t nout, int64_t max_delay) {
+    // delay spreads of a stage are held against its mean (the widest stages of a dispersion sweep
+    // run 1.4-1.6 times that)
+    const int64_t wide_sum = max_delay * gulp_swar_stage_channels(nbits, GulpForm::wide);
+    const bool lengthy = aligned && nchans * nbits / 8 * nout >= 100000000;  // blocks enough, though each does twice the work
+    if (nbits == 2 && lengthy && wide_sum <= Geo<2, GulpForm::wide>::SPREAD * nchans) return GulpForm::wide;
+    if (nbits == 8 && lengthy && 2 * wide_sum <= Geo<8, GulpForm::wide>::SPREAD * nchans) return GulpForm::wide;
+    if (nbits < 4) return GulpForm::normal;
+    const int64_t spread = nbits == 8 ? Geo<8, GulpForm::compact>::SPREAD : Geo<4, GulpForm::compact>::SPREAD;
+    return 2 * max_delay * gulp_swar_stage_channels(nbits, GulpForm::compact) <= spread * nchans ? GulpForm::compact
+                                                                                                 : GulpForm::normal;
+}
 
-bool gulp_swar_applies(const void* in, int nbits, int64_t nchans) {
-    if (nbits != 1 && nbits != 2 && nbits != 4 && nbits != 8) return false;
-    return (nchans * nbits) % 32 == 0 && reinterpret_cast<uintptr_t>(in) % 4 == 0;
+bool gulp_swar_applies(int nbits, int64_t nchans) {
+    return (nbits == 1 || nbits == 2 || nbits == 4 || nbits == 8) && nchans * nbits >= 32;
 }
 
 int launch_gulp_swar(const uint8_t* in, int nbits, bool big, const int32_t* delays, float* out, int64_t nchans,
                      int64_t nsamps, int64_t nout, int64_t out_start, int64_t row_bytes, int64_t chans_per_group,
-                     int64_t groups, int64_t ilv, int64_t nchunk, int use_atomic, bool compact, hipStream_t st) {
+                     int64_t groups, int64_t ilv, int64_t nchunk, int use_atomic, GulpForm form, hipStream_t st) {
     SPP_REQUIRE(chans_per_group * nchunk <= swar_max_channels(nbits), "too many channels per block");
-    SPP_REQUIRE(!compact || nbits >= 4, "the compact form is for 4- and 8-bit data");
+    const bool aligned = row_bytes % 4 == 0 && reinterpret_cast<uintptr_t>(in) % 4 == 0;
     const int64_t bx = ceil_div(nout, gulp_swar_tile(nbits));
     const int64_t nblocks = bx * groups;
     SPP_REQUIRE(nblocks <= 0x7ffffff0LL, "gulp too long");
     const dim3 grid(static_cast<unsigned>(ceil_div(nblocks, int64_t(8)) * 8));
-#define SPP_SWAR(NB, BG, CP)                                                                                   \
-    hipLaunchKernelGGL((k_gulp_swar<NB, BG, CP>), grid, dim3(GS_THREADS), 0, st, in, delays, out, nchans, nsamps, \
-                       nout, out_start, row_bytes, chans_per_group, groups, nblocks, ilv, nchunk, use_atomic)
-    switch (nbits * 4 + (big && nbits < 8 ? 2 : 0) + (compact ? 1 : 0)) {  // bit order: sub-byte samples only
-        case 4: SPP_SWAR(1, false, false); break;
-        case 6: SPP_SWAR(1, true, false); break;
-        case 8: SPP_SWAR(2, false, false); break;
-        case 10: SPP_SWAR(2, true, false); break;
-        case 16: SPP_SWAR(4, false, false); break;
-        case 17: SPP_SWAR(4, false, true); break;
-        case 18: SPP_SWAR(4, true, false); break;
-        case 19: SPP_SWAR(4, true, true); break;
-        case 33: SPP_SWAR(8, false, true); break;
-        default: SPP_SWAR(8, false, false); break;
+#define SPP_SWAR1(NB, BG, FM, AL)                                                                                     \
+    hipLaunchKernelGGL((k_gulp_swar<NB, BG, GulpForm::FM, AL>), grid, dim3(Geo<NB, GulpForm::FM>::THREADS), 0, st, in, \
+                       delays, out, nchans, nsamps, nout, out_start, row_bytes, chans_per_group, groups, nblocks, ilv, \
+                       nchunk, use_atomic)
+#define SPP_SWAR(NB, BG, FM)                       \
+    do {                                           \
+        if (aligned) SPP_SWAR1(NB, BG, FM, true);  \
+        else SPP_SWAR1(NB, BG, FM, false);         \
+    } while (0)
+    const bool compact = form == GulpForm::compact, wide = form == GulpForm::wide;
+    SPP_REQUIRE(aligned || !wide, "the wide form takes rows of whole dwords");
+    switch (nbits * 2 + (big && nbits < 8 ? 1 : 0)) {  // bit order: sub-byte samples only
+        case 2: SPP_SWAR(1, false, normal); break;
+        case 3: SPP_SWAR(1, true, normal); break;
+        case 4: if (wide) SPP_SWAR1(2, false, wide, true); else SPP_SWAR(2, false, normal); break;
+        case 5: if (wide) SPP_SWAR1(2, true, wide, true); else SPP_SWAR(2, true, normal); break;
+        case 8: if (compact) SPP_SWAR(4, false, compact); else SPP_SWAR(4, false, normal); break;
+        case 9: if (compact) SPP_SWAR(4, true, compact); else SPP_SWAR(4, true, normal); break;
+        default:
+            if (wide) SPP_SWAR1(8, false, wide, true);
+            else if (compact) SPP_SWAR(8, false, compact);
+            else SPP_SWAR(8, false, normal);
     }
+#undef SPP_SWAR1
 #undef SPP_SWAR
     SPP_LAUNCHED("k_gulp_swar");
     return SPP_OK;

@@ -1,5 +1,5 @@
 // One-DM dedispersion of packed 1/2/4/8-bit gulps with word-parallel (SWAR) adds: the
-// dedisperse form of spp_dedisperse, used when each packed row is whole dwords.
+// dedisperse form of spp_dedisperse, for rows of at least four bytes.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -8,9 +8,12 @@
 
 namespace spp {
 
-// True when the SWAR kernel takes this launch: 1/2/4/8-bit rows of whole dwords on a 4-byte
-// aligned stream.
-bool gulp_swar_applies(const void* in, int nbits, int64_t nchans);
+// Block forms of the kernel (gulp_swar.hip): narrow stages with the full or a compact series buffer,
+// or wide stages.
+enum class GulpForm { normal, compact, wide };
+
+// True when the SWAR kernel takes this launch: 1/2/4/8-bit rows of at least 4 bytes.
+bool gulp_swar_applies(int nbits, int64_t nchans);
 
 // out[out_start + t] (t < nout) = sum over channels of x[t + delays[c]][c], with x[row] for
 // row < 0 taken from row + nsamps and rows >= nsamps read as 0 (only outputs t >= nout reach
@@ -19,16 +22,16 @@ bool gulp_swar_applies(const void* in, int nbits, int64_t nchans);
 // zeroed output. Returns an SPP_* status.
 int launch_gulp_swar(const uint8_t* in, int nbits, bool big, const int32_t* delays, float* out, int64_t nchans,
                      int64_t nsamps, int64_t nout, int64_t out_start, int64_t row_bytes, int64_t chans_per_group,
-                     int64_t groups, int64_t ilv, int64_t nchunk, int use_atomic, bool compact, hipStream_t st);
+                     int64_t groups, int64_t ilv, int64_t nchunk, int use_atomic, GulpForm form, hipStream_t st);
 
 // Outputs per block for nbits (the time tile).
 int64_t gulp_swar_tile(int nbits);
 
-// True when the compact form (a smaller series buffer: more blocks per CU, fewer rows per pass)
-// suits a launch whose largest delay is max_delay (4/8-bit data only).
-bool gulp_swar_compact(int nbits, int64_t nchans, int64_t max_delay);
+// The block form that suits a launch whose largest delay is max_delay; aligned: rows of whole dwords
+// on a 4-byte aligned stream.
+GulpForm gulp_swar_form(int nbits, bool aligned, int64_t nchans, int64_t nout, int64_t max_delay);
 
-// Channels per stage for nbits (a stage is a fixed run of dwords of each row).
-int64_t gulp_swar_stage_channels(int nbits);
+// Channels per stage (a stage is a fixed run of dwords of each row).
+int64_t gulp_swar_stage_channels(int nbits, GulpForm form);
 
 }  // namespace spp
