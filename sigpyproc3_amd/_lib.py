@@ -217,6 +217,51 @@ def to_device(a: np.ndarray):
     return t.from_numpy(a).to(device(), non_blocking=False)
 
 
+# Results of this size and up come to the host through pinned staging: a pageable copy of 16 MiB
+# runs at 17 GB/s here, two 2 MiB pinned buffers and a threaded copy out of them at 36 (4 MiB 16 and
+# 32, 1 MiB level; 512 KiB buffers give no gain, 4 MiB ones no more).
+STAGE_BYTES = 2 << 20
+_STAGED_MIN = STAGE_BYTES
+
+_staging = threading.local()  # .buffers: this thread's two pinned buffers, freed when it ends
+
+
+def to_host(x) -> np.ndarray:
+    """A device tensor's values in a new pageable host array (waits for the current stream's copy).
+
+    Large tensors arrive in pieces: while one pinned buffer is filled by the device, torch's
+    CPU threads copy the other into the result (which also spreads its page faults).
+    """
+    t = torch()
+    nbytes = int(x.numel()) * x.element_size()
+    if nbytes < _STAGED_MIN or not x.is_cuda:
+        return x.cpu().numpy()
+    if not hasattr(_staging, "buffers"):
+        try:
+            _staging.buffers = [t.empty(STAGE_BYTES, dtype=t.uint8, pin_memory=True) for _ in range(2)]
+        except RuntimeError:  # no pinned memory to be had
+            return x.cpu().numpy()
+    src = x.contiguous().reshape(-1).view(t.uint8)
+    out = t.empty(tuple(x.shape), dtype=x.dtype)
+    dst = out.reshape(-1).view(t.uint8)
+    with t.cuda.device(x.device):
+        arrived = [t.cuda.Event(), t.cuda.Event()]
+        pieces = [(a, min(a + STAGE_BYTES, nbytes)) for a in range(0, nbytes, STAGE_BYTES)]
+
+        def drain(k: int) -> None:
+            a, b = pieces[k]
+            arrived[k & 1].synchronize()
+            dst[a:b].copy_(_staging.buffers[k & 1][: b - a])
+
+        for k, (a, b) in enumerate(pieces):
+            _staging.buffers[k & 1][: b - a].copy_(src[a:b], non_blocking=True)
+            arrived[k & 1].record()
+            if k > 0:
+                drain(k - 1)
+        drain(len(pieces) - 1)
+    return out.numpy()
+
+
 def empty(shape, dtype: str):
     t = torch()
     return t.empty(shape, dtype=getattr(t, dtype), device=device())

@@ -182,7 +182,7 @@ class Filterbank(ABC):
         for nsamps_r, ii, dev, _nb in self._device_gulps(gulp, start, nsamps, plan_kwargs, max_delay):
             _lib.call("spp_dedisperse", _lib.ptr(dev), nbits, big, hdr.nchans, nsamps_r,
                       _lib.ptr(d_dev), max_delay, _lib.ptr(tim), ii * (gulp - max_delay), stream)
-        data = tim[:tim_len].cpu().numpy() if tim_len > 0 else np.zeros(0, dtype=np.float32)
+        data = _lib.to_host(tim[:tim_len]) if tim_len > 0 else np.zeros(0, dtype=np.float32)
         return TimeSeries(data, hdr.new_header({"nchans": 1, "dm": dm, "nsamples": tim_len}))
 
     def subband(self, dm: float, nsub: int, ref_freq: str | float = "fch1",
@@ -218,7 +218,7 @@ class Filterbank(ABC):
                           _lib.ptr(d_dev), _lib.ptr(cts_dev), max_delay, nsub, _lib.ptr(out_dev),
                           out_len, stream)
                 nwrite = (nsamps_r - max_delay) * nsub
-                out_file.cwrite(out_dev[:nwrite].cpu().numpy())
+                out_file.cwrite(_lib.to_host(out_dev[:nwrite]))
         finally:
             out_file.close()
         return outfile_name
@@ -265,7 +265,7 @@ class Filterbank(ABC):
                 raise ValueError(msg)
             _lib.call("spp_collapse", _lib.ptr(dev), nbits, big, hdr.nchans, nsamps_r, _lib.ptr(tim),
                       ii * nsamps_r, stream)
-        tim_ar = tim[:tim_len].cpu().numpy() if tim_len > 0 else np.zeros(0, dtype=np.float32)
+        tim_ar = _lib.to_host(tim[:tim_len]) if tim_len > 0 else np.zeros(0, dtype=np.float32)
         if method == "mean":
             tim_ar /= hdr.nchans
         return TimeSeries(tim_ar, hdr.new_header({"nchans": 1, "dm": 0}))
@@ -356,7 +356,7 @@ class Filterbank(ABC):
             for _nr, _ii, dev, nb in self._device_gulps(gulp, start, nsamps, plan_kwargs):
                 _lib.call("spp_mask_bytes", _lib.ptr(dev), nb, self.samp_stride, _lib.ptr(keep_d),
                           _lib.ptr(set_d), stream)
-                out_file.write(dev[:nb].cpu().numpy().tobytes())
+                out_file.write(_lib.to_host(dev[:nb]).tobytes())
         finally:
             out_file.close()
         return outfile_name
@@ -388,7 +388,7 @@ class Filterbank(ABC):
             for nsamps_r, _ii, dev, _nb in self._device_gulps(gulp, start, nsamps, plan_kwargs):
                 _lib.call("spp_remove_zerodm", _lib.ptr(dev), nbits, big, hdr.nchans, nsamps_r,
                           _lib.ptr(w_d), _lib.ptr(b_d), _lib.ptr(out_dev), stream)
-                out_file.cwrite(out_dev[: nsamps_r * hdr.nchans].cpu().numpy())
+                out_file.cwrite(_lib.to_host(out_dev[: nsamps_r * hdr.nchans]))
         finally:
             out_file.close()
         return outfile_name

@@ -163,7 +163,7 @@ def _run_roll(data: np.ndarray, off: np.ndarray, width: int) -> np.ndarray:
         r1 = min(nrows, r0 + 65535)
         _lib.call("spp_roll_rows", _lib.ptr(src[r0:r1]), r1 - r0, ncols, _lib.ptr(off_h[r0:r1]),
                   _lib.ptr(off_d[r0:r1]), width, _lib.ptr(out[r0:r1]), _lib.stream_handle())
-    return out.cpu().numpy()
+    return _lib.to_host(out)
 
 
 def _run_dmt(data: np.ndarray, off: np.ndarray, width: int) -> np.ndarray:
@@ -178,4 +178,4 @@ def _run_dmt(data: np.ndarray, off: np.ndarray, width: int) -> np.ndarray:
         i1 = min(ndm, i0 + 65535)
         _lib.call("spp_dmt", _lib.ptr(src), nchans, ncols, _lib.ptr(off_h[i0:i1]), _lib.ptr(off_d[i0:i1]),
                   i1 - i0, width, _lib.ptr(out[i0:i1]), _lib.stream_handle())
-    return out.cpu().numpy()
+    return _lib.to_host(out)

@@ -41,7 +41,7 @@ def _unpack(array, unpacked, nbits: int, big: int) -> None:
     dst = _lib.empty((n * (8 // nbits),), "uint8") if host_out else unpacked
     _lib.call("spp_unpack", _lib.ptr(src), n, _lib.ptr(dst), nbits, big, _lib.stream_handle())
     if host_out:
-        unpacked[:] = dst.cpu().numpy()
+        unpacked[:] = _lib.to_host(dst)
 
 
 # kernels.unpack{1,2,4}_8_{big,little} (core/kernels.py:20-69)
@@ -104,7 +104,7 @@ def dedisperse(in_arr, out_arr, delays, nchans: int, nsamps: int, out_start_inde
     _lib.call("spp_dedisperse", _lib.ptr(src), nbits, 0, nchans, nsamps, _lib.ptr(d), md,
               _lib.ptr(base), start, _lib.stream_handle())
     if host_out:
-        out_arr[out_start_index : out_start_index + nout] = dst.cpu().numpy()
+        out_arr[out_start_index : out_start_index + nout] = _lib.to_host(dst)
 
 
 # The reference's parallel variant (core/kernels.py:542) computes the same values.
@@ -134,7 +134,7 @@ def subband(inarray, outarray, delays, chan_to_sub, maxdelay: int, nchans: int, 
     _lib.call("spp_subband", _lib.ptr(src), 32 if is_f32 else 8, 0, nchans, nsamps, _lib.ptr(d),
               _lib.ptr(cts), maxdelay, nsubs, _lib.ptr(dst), size, _lib.stream_handle())
     if host_out:
-        outarray[:] = dst.cpu().numpy()
+        outarray[:] = _lib.to_host(dst)
 
 
 def good_size_real(n: int) -> int:
@@ -196,4 +196,4 @@ def convolve_templates(data, temp_bank, ref_bin) -> np.ndarray:
     _lib.call("spp_convolve_templates", _lib.ptr(src), n, _lib.ptr(taps), _lib.ptr(lens),
               _lib.ptr(refs), len(temps), _lib.ptr(convs), _lib.ptr(ws), int(need[0]),
               _lib.stream_handle())
-    return convs.cpu().numpy()
+    return _lib.to_host(convs)

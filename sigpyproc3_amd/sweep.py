@@ -228,7 +228,7 @@ def dedisperse_resident(packed, header, dm: float, ref_freq: str | float = "fch1
             _lib.call("spp_dedisperse", _lib.ptr(packed[pos * row_bytes :]), nbits, big, hdr.nchans, nr,
                       _lib.ptr(d_dev), md, _lib.ptr(tim), ii * (gulp - md), st)
             pos += nr + skip
-    data = tim[:tim_len].cpu().numpy() if tim_len > 0 else np.zeros(0, dtype=np.float32)
+    data = _lib.to_host(tim[:tim_len]) if tim_len > 0 else np.zeros(0, dtype=np.float32)
     return TimeSeries(data, hdr.new_header({"nchans": 1, "dm": dm, "nsamples": tim_len}))
 
 
@@ -249,7 +249,7 @@ def running_normalise(x, row_len, window: int = 4096, *, ld: int | None = None, 
     ws = _lib.empty((int(need[0]),), "uint8")
     _lib.call("spp_running_normalise", _lib.ptr(xd), ldx, nrows, _lib.ptr(rl), int(window),
               _lib.ptr(z), int(z.shape[1]), _lib.ptr(ws), int(need[0]), _lib.stream_handle(stream))
-    return z.cpu().numpy() if host else z
+    return _lib.to_host(z) if host else z
 
 
 def normalise_boxcar_mf(x, row_len, window: int = 4096, widths=DEFAULT_WIDTHS, *, stream=None):
@@ -314,7 +314,7 @@ class SweepResult:
         return int(self.plane.shape[0])
 
     def row(self, i: int) -> np.ndarray:
-        return self.plane[i, : int(self.row_len[i])].cpu().numpy()
+        return _lib.to_host(self.plane[i, : int(self.row_len[i])])
 
     def timeseries(self, i: int):
         """Row ``i`` as the ``TimeSeries`` ``Filterbank.dedisperse(dms[i])`` returns."""
