@@ -101,11 +101,12 @@ int spp_sweep_plan_create(const int32_t* table_host, int64_t ndm, int64_t nchans
 int spp_sweep_plan_destroy(spp_sweep_plan* plan);
 /* Block shapes of the stage-2 kernel (DM rows per wave x waves x channels per stage):
  * 1/2-bit data: 0 = 2x8x16, 1 = 2x8x20, 2 = 2x8x8 (6 waves per SIMD), 3 = 2x8x12 (6 waves per
- *               SIMD), 4 = 1x16x16 (8 waves per SIMD, default), 5 = 1x16x12 (8 waves per SIMD);
- * 4/8-bit data: 0 = 2x8x12 (6 waves per SIMD, default), 1 = 2x8x16, 2 = 4x4x8, 3 = 2x8x8,
- *               4 = 1x16x16, 5 = 1x16x12 (8 waves per SIMD).
- * All give identical results; spp_sweep_plan_set_variant picks one for a plan (the
- * autotuner times them). */
+ *               SIMD), 4 = 1x16x16 (8 waves per SIMD), 5 = 1x16x12 (8 waves per SIMD),
+ *               6 = 1x8x32 (blocks of 8 rows);
+ * 4/8-bit data: 0 = 2x8x12 (6 waves per SIMD), 1 = 2x8x16, 2 = 4x4x8, 3 = 2x8x8,
+ *               4 = 1x16x16, 5 = 1x16x12 (8 waves per SIMD), 6 = 1x8x16 (4-bit) or 1x8x32.
+ * All give identical results. Each execution takes the shape that suits its size unless
+ * spp_sweep_plan_set_variant has picked one for the plan (the autotuner times them). */
 int spp_sweep_variant_count(void);
 int spp_sweep_plan_set_variant(spp_sweep_plan* plan, int variant);
 int spp_sweep_plan_info(const spp_sweep_plan* plan, spp_sweep_info* info);

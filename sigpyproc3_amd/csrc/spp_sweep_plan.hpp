@@ -15,7 +15,8 @@ struct spp_sweep_plan {
     int64_t max_len = 0, min_len = 0, total = 0;
     int32_t max_spread = 0;
     bool use32 = false;
-    int variant = 0;  // k_sweep block shape (launch_sweep)
+    int variant = 0;  // k_sweep block shape (launch_sweep): set by the caller, or else picked per execution
+    bool variant_set = false;
     int64_t gpitch = 0;
     std::vector<uint8_t> relw;   // [ndm][rpitch] = delay - tile base (rounded down to 4) < 256
     int64_t rpitch = 0;          // bytes per row: nchans + 64 rounded up to 16; zero past nchans

@@ -63,6 +63,28 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(MINW
 
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
+// The block shape of an execution whose longest row has max_len samples (launch_sweep lists them),
+// by its count of 16-row blocks. Measured (us of k_sweep):
+//   <= 128 blocks: half the CUs or more would hold no 16-row block, so blocks of 8 rows; one fits a
+//     CU, so it may take 128 KB of LDS, and 32 channels a stage halve the barriers. 1-bit 336
+//     channels x 20011, 64 rows: 25 (34 with 16 rows); 2-bit 4096 x 20000, 64 rows: 268 (353); 8-bit
+//     1024 x 40000, 40 rows, 120 blocks: 89 (116). Past 128 some CUs run two: 8-bit 141 blocks 131
+//     against 116, 2-bit 150 blocks 110 against 95;
+//   4-bit: 8 channels a stage, 2 rows a wave in full grids (4096 x 2^18, 512 rows: 8740, against
+//     9290 one row a wave and 9540 with 12 channels; 336 x 120000, 200 rows, 1534 blocks: 156 against
+//     159 and 165), one row a wave up to 1024 blocks (944 blocks: 311 against 315 and 339);
+//   8-bit: one row a wave (4096 x 60000, 128 rows: 1440, against 1540 with two rows and 12 channels;
+//     1024 x 2^19, 512 rows, 16384 blocks: 5570 against 5800); the two meet at 4096 x 2^18, 512 rows,
+//     and two rows win by 1 % above (4096 x 2^19, 1024 rows, 32768 blocks: 44200 against 44600).
+int auto_variant(const spp_sweep_plan* p, int64_t max_len) {
+    const int64_t T = (p->nbits <= 2 ? 8 : 4) * SW_S;
+    const int64_t blocks = static_cast<int64_t>(p->tile_dm0.size()) * spp::ceil_div(max_len, T);
+    if (blocks <= 128) return 6;
+    if (p->nbits <= 2) return 4;
+    if (p->nbits == 4) return blocks <= 1024 ? 4 : 3;
+    return blocks <= 16384 ? 4 : 0;
+}
+
 }  // namespace
 
 
@@ -151,9 +173,7 @@ extern "C" int spp_sweep_plan_create(const int32_t* table_host, int64_t ndm, int
         i = j;
     }
     p->use32 = static_cast<int64_t>(nchans) * maxv > 65535;
-    // Nibble data: 16 waves x 1 DM row x 16 channels per stage at 8 waves per SIMD (variant 4);
-    // byte data: 8 waves x 2 DM rows x 12 channels at 6 waves per SIMD (variant 0); tunable
-    p->variant = nbits <= 2 ? 4 : 0;
+    p->variant = auto_variant(p, p->max_len);
     p->gpitch = ((nsamps + 63) / 64) * 64;
     const int64_t ntiles = static_cast<int64_t>(p->tile_dm0.size());
     int64_t off = 0;
@@ -169,7 +189,7 @@ extern "C" int spp_sweep_plan_create(const int32_t* table_host, int64_t ndm, int
     return SPP_OK;
 }
 
-extern "C" int spp_sweep_variant_count(void) { return 6; }
+extern "C" int spp_sweep_variant_count(void) { return 7; }
 
 extern "C" int spp_sweep_plan_set_variant(spp_sweep_plan* p, int variant) {
     spp::clear_error();
@@ -177,6 +197,7 @@ extern "C" int spp_sweep_plan_set_variant(spp_sweep_plan* p, int variant) {
     SPP_REQUIRE(variant >= 0 && variant < spp_sweep_variant_count(), "variant %d outside [0, %d)", variant,
                 spp_sweep_variant_count());
     p->variant = variant;
+    p->variant_set = true;
     return SPP_OK;
 }
 
@@ -295,26 +316,29 @@ int launch_sweep_v(const spp_sweep_plan* p, const Extent& e, char* ws, float* pl
 // The kernel is bound by its LDS reads. One DM row per wave in 16-wave blocks holds the
 // accumulators of one row (about 60 VGPRs, no spills) and so runs 8 waves per SIMD; with 16
 // channels per stage (64 KB of LDS, two blocks per CU) it is the fastest shape measured for
-// nibble data and on a par with the 2 x 8 x 12 shape for byte data.
+// nibble data; auto_variant says where another one is taken.
 template <int NBITS, bool USE32>
 int launch_sweep(const spp_sweep_plan* p, const Extent& e, char* ws, float* plane, int64_t ld,
                  hipStream_t st) {
+    const int variant = p->variant_set ? p->variant : auto_variant(p, e.max_len);
     if constexpr (NBITS <= 2) {
-        switch (p->variant) {
+        switch (variant) {
             case 1: return launch_sweep_v<NBITS, USE32, 2, 8, 20, 4>(p, e, ws, plane, ld, st);
             case 2: return launch_sweep_v<NBITS, USE32, 2, 8, 8, 6>(p, e, ws, plane, ld, st);
             case 3: return launch_sweep_v<NBITS, USE32, 2, 8, 12, 6>(p, e, ws, plane, ld, st);
             case 4: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8>(p, e, ws, plane, ld, st);
             case 5: return launch_sweep_v<NBITS, USE32, 1, 16, 12, 8>(p, e, ws, plane, ld, st);
+            case 6: return launch_sweep_v<NBITS, USE32, 1, 8, 32, 2>(p, e, ws, plane, ld, st);
             default: return launch_sweep_v<NBITS, USE32, 2, 8, 16, 4>(p, e, ws, plane, ld, st);
         }
     } else {
-        switch (p->variant) {
+        switch (variant) {
             case 1: return launch_sweep_v<NBITS, USE32, 2, 8, 16, 4>(p, e, ws, plane, ld, st);
             case 2: return launch_sweep_v<NBITS, USE32, 4, 4, 8, 3>(p, e, ws, plane, ld, st);
             case 3: return launch_sweep_v<NBITS, USE32, 2, 8, 8, 4>(p, e, ws, plane, ld, st);
             case 4: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8>(p, e, ws, plane, ld, st);
             case 5: return launch_sweep_v<NBITS, USE32, 1, 16, 12, 8>(p, e, ws, plane, ld, st);
+            case 6: return launch_sweep_v<NBITS, USE32, 1, 8, (NBITS == 4 ? 16 : 32), 2>(p, e, ws, plane, ld, st);
             default: return launch_sweep_v<NBITS, USE32, 2, 8, 12, 6>(p, e, ws, plane, ld, st);
         }
     }
