@@ -36,7 +36,7 @@ __global__ __launch_bounds__(B_THREADS) void k_build_g(const uint8_t* __restrict
 
 // Stage 2: one block per (time tile, DM tile, sub-tile of K * WAVES rows). XCD-aware order:
 // consecutive blocks on one XCD walk the DM tiles of one time tile.
-template <int NBITS, bool USE32, int K, int WAVES, int CC, int MINW>
+template <int NBITS, bool USE32, int K, int WAVES, int CC, int MINW, bool SKIP>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(MINW))) void k_sweep(
     const uint32_t* __restrict__ G, int64_t gpitch, int64_t glen, int64_t nchans,
     const uint32_t* __restrict__ relw4, int64_t rpitch4, const int32_t* __restrict__ basew,
@@ -70,6 +70,10 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 //     channels x 20011, 64 rows: 25 (34 with 16 rows); 2-bit 4096 x 20000, 64 rows: 268 (353); 8-bit
 //     1024 x 40000, 40 rows, 120 blocks: 89 (116). Past 128 some CUs run two: 8-bit 141 blocks 131
 //     against 116, 2-bit 150 blocks 110 against 95;
+//   tiles at most 4/5 full (rows whose delays lie far apart): one row a wave, the waves without a row
+//     skip the sums. 256 rows of 1024 channels x 2^17 in 29 tiles, 1 / 2 / 4 / 8-bit: 389 426 824 1007
+//     (535 553 1114 1320 with sums over padding rows; best other shape at 4-bit 1060); in 52 tiles
+//     545 564 1120 1322 (855 882 1799 2262). At 18 tiles 360 358 698 842 against 350 362 661 802;
 //   4-bit: 8 channels a stage, 2 rows a wave in full grids (4096 x 2^18, 512 rows: 8740, against
 //     9290 one row a wave and 9540 with 12 channels; 336 x 120000, 200 rows, 1534 blocks: 156 against
 //     159 and 165), one row a wave up to 1024 blocks (944 blocks: 311 against 315 and 339);
@@ -80,6 +84,7 @@ int auto_variant(const spp_sweep_plan* p, int64_t max_len) {
     const int64_t T = (p->nbits <= 2 ? 8 : 4) * SW_S;
     const int64_t blocks = static_cast<int64_t>(p->tile_dm0.size()) * spp::ceil_div(max_len, T);
     if (blocks <= 128) return 6;
+    if (p->ndm * 5 <= static_cast<int64_t>(p->tile_dm0.size()) * SW_DT * 4) return 7;
     if (p->nbits <= 2) return 4;
     if (p->nbits == 4) return blocks <= 1024 ? 4 : 3;
     return blocks <= 16384 ? 4 : 0;
@@ -189,7 +194,7 @@ extern "C" int spp_sweep_plan_create(const int32_t* table_host, int64_t ndm, int
     return SPP_OK;
 }
 
-extern "C" int spp_sweep_variant_count(void) { return 7; }
+extern "C" int spp_sweep_variant_count(void) { return 8; }
 
 extern "C" int spp_sweep_plan_set_variant(spp_sweep_plan* p, int variant) {
     spp::clear_error();
@@ -291,7 +296,7 @@ int launch_build(const uint8_t* packed, const spp_sweep_plan* p, const Extent& e
     return SPP_OK;
 }
 
-template <int NBITS, bool USE32, int K, int WAVES, int CC, int MINW>
+template <int NBITS, bool USE32, int K, int WAVES, int CC, int MINW, bool SKIP = false>
 int launch_sweep_v(const spp_sweep_plan* p, const Extent& e, char* ws, float* plane, int64_t ld,
                    hipStream_t st) {
     const int64_t ntiles_dm = static_cast<int64_t>(p->tile_dm0.size());
@@ -299,7 +304,7 @@ int launch_sweep_v(const spp_sweep_plan* p, const Extent& e, char* ws, float* pl
     const int64_t nblocks = ntiles_dm * (SW_DT / (K * WAVES)) * ntiles_t;
     const int64_t grid = spp::ceil_div(nblocks, 8) * 8;
     SPP_REQUIRE(grid <= 0x7fffffffLL, "sweep grid too large");
-    hipLaunchKernelGGL((k_sweep<NBITS, USE32, K, WAVES, CC, MINW>), dim3(static_cast<unsigned>(grid)),
+    hipLaunchKernelGGL((k_sweep<NBITS, USE32, K, WAVES, CC, MINW, SKIP>), dim3(static_cast<unsigned>(grid)),
                        dim3(WAVES * 64), 0, st, e.G, e.gpitch, e.glen, p->nchans, reinterpret_cast<const uint32_t*>(ws + p->off_relw),
                        p->rpitch / 4, reinterpret_cast<const int32_t*>(ws + p->off_base),
                        reinterpret_cast<const int32_t*>(ws + p->off_dm0),
@@ -328,6 +333,7 @@ int launch_sweep(const spp_sweep_plan* p, const Extent& e, char* ws, float* plan
             case 3: return launch_sweep_v<NBITS, USE32, 2, 8, 12, 6>(p, e, ws, plane, ld, st);
             case 4: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8>(p, e, ws, plane, ld, st);
             case 5: return launch_sweep_v<NBITS, USE32, 1, 16, 12, 8>(p, e, ws, plane, ld, st);
+            case 7: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8, true>(p, e, ws, plane, ld, st);
             case 6: return launch_sweep_v<NBITS, USE32, 1, 8, 32, 2>(p, e, ws, plane, ld, st);
             default: return launch_sweep_v<NBITS, USE32, 2, 8, 16, 4>(p, e, ws, plane, ld, st);
         }
@@ -338,6 +344,7 @@ int launch_sweep(const spp_sweep_plan* p, const Extent& e, char* ws, float* plan
             case 3: return launch_sweep_v<NBITS, USE32, 2, 8, 8, 4>(p, e, ws, plane, ld, st);
             case 4: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8>(p, e, ws, plane, ld, st);
             case 5: return launch_sweep_v<NBITS, USE32, 1, 16, 12, 8>(p, e, ws, plane, ld, st);
+            case 7: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8, true>(p, e, ws, plane, ld, st);
             case 6: return launch_sweep_v<NBITS, USE32, 1, 8, (NBITS == 4 ? 16 : 32), 2>(p, e, ws, plane, ld, st);
             default: return launch_sweep_v<NBITS, USE32, 2, 8, 12, 6>(p, e, ws, plane, ld, st);
         }

@@ -19,18 +19,11 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("nbits,nchans,ndm,blocks", CASES)
-def test_default_shape(nbits, nchans, ndm, blocks):
+def _check(rng, table, nsamps, nbits, tiles):
     from sigpyproc3_amd import _lib
     from sigpyproc3_amd.sweep import SweepPlan
 
-    rng = np.random.default_rng(nbits * 1000 + blocks)
-    T = 2048 if nbits <= 2 else 1024
-    # per-row delays rise by a sample per row over the band; the rows share DM tiles of 16
-    table = (np.arange(ndm)[:, None] * np.linspace(0, 1, nchans)[None, :]).astype(np.int32)
-    table[:, -1] = np.arange(ndm)
-    tiles = -(-ndm // 16)
-    nsamps = (blocks // tiles) * T - T // 2
+    ndm, nchans = table.shape
     order = O.DEFAULT_BITORDER.get(nbits, "big")
     samples = rng.integers(0, 1 << nbits, nsamps * nchans, dtype=np.uint8)
     packed = samples if nbits == 8 else O.pack(samples, nbits, order)
@@ -43,3 +36,23 @@ def test_default_shape(nbits, nchans, ndm, blocks):
         n = int(plan.row_len[i])
         np.testing.assert_array_equal(plane[i, :n], ref[i, :n], err_msg=f"row {i}")
         assert not plane[i, n:].any()
+
+
+@pytest.mark.parametrize("nbits,nchans,ndm,blocks", CASES)
+def test_default_shape(nbits, nchans, ndm, blocks):
+    T = 2048 if nbits <= 2 else 1024
+    # delays rise by a sample a row at the band's far end; 16 rows share a DM tile
+    table = (np.arange(ndm)[:, None] * np.linspace(0, 1, nchans)[None, :]).astype(np.int32)
+    tiles = -(-ndm // 16)
+    _check(np.random.default_rng(nbits * 1000 + blocks), table, (blocks // tiles) * T - T // 2, nbits, tiles)
+
+
+@pytest.mark.parametrize("nbits", [1, 2, 4, 8])
+@pytest.mark.parametrize("step,per_tile", [(60, 5), (250, 2), (300, 1), (17, 15), (20, 13)])
+def test_tiles_with_few_rows(nbits, step, per_tile):
+    # tiles hold the rows within 252 samples; each row ends `step` samples before the last, so whole
+    # blocks of some rows lie past their ends
+    ndm, nchans, T = 41, 40, 2048 if nbits <= 2 else 1024
+    table = np.round(step * np.arange(ndm)[:, None] * np.linspace(0, 1, nchans)[None, :]).astype(np.int32)
+    tiles = -(-ndm // per_tile)
+    _check(np.random.default_rng(nbits * 1000 + step), table, (128 // tiles + 12) * T + 333, nbits, tiles)
