@@ -2,7 +2,7 @@
 // persistent kernel launch over a device work queue.
 //
 // The queue is a sequence of segments. A round is a set of instances whose stage-1 copies G
-// fit one G pool; each round has a stage-1 segment B_r (items: B_TJ words x BATCH_BCW packed
+// fit one G pool; each round has a stage-1 segment B_r (items: B_TJ words x batch_bcw() packed
 // bytes of one instance) and a stage-2 segment S_r (items: D DM rows x ntt time tiles of one
 // instance). With R rounds the order is
 //   B_0, B_1, S_0, S_1, B_2, B_3, S_2, S_3, B_4, ...
@@ -37,7 +37,12 @@ namespace {
 constexpr int BQ = 8;                       // sub-queues per segment (one per XCD)
 constexpr int BT_RUN = 4;                   // consecutive time-tile groups per sub-queue run
 constexpr int BB_RUN = 32;                  // consecutive stage-1 time blocks per sub-queue run
-constexpr int BATCH_BCW = 32;               // packed bytes per row of a stage-1 item
+// Packed bytes per row of a stage-1 item, for a block shape of CC channels per stage: 64 use half a
+// 128-byte line of the stream at a time and 70 KB of LDS, which the shapes of 16 channels (64 KB,
+// two blocks per CU) have room for; the smaller shapes hold more blocks per CU with 32. Batches of
+// 6, 12 and 16 uneven sweeps in the default shape: 8.59 3.75 7.44 ms with 32, 7.73 3.48 6.74 with
+// 64 (7.83 3.48 6.67 with 32 loads in flight, 7.82 3.50 6.74 with 8).
+constexpr int batch_bcw(int cc) { return cc >= 16 ? 64 : 32; }
 constexpr int BATCH_LOADS = 16;             // stage-1 staging loads in flight per thread
 constexpr uint32_t SPIN_LIMIT = 1u << 24;   // polls (about 0.2 us each) before a wait fails
 constexpr int NSHAPES = 5;
@@ -130,27 +135,27 @@ __device__ __forceinline__ int opaque_tid() {
     return t;
 }
 
-template <int NBITS, bool BIG, int NT>
+template <int NBITS, bool BIG, int NT, int BCW>
 __device__ __forceinline__ void build_item(CInst& in, int64_t j0, int64_t b0, uint8_t* raw) {
     if (in.aligned)
-        build_tile<NBITS, BIG, true, BATCH_BCW, BATCH_LOADS, NT>(glob(in.packed), in.nsamps, in.nchans, glob(in.G),
+        build_tile<NBITS, BIG, true, BCW, BATCH_LOADS, NT>(glob(in.packed), in.nsamps, in.nchans, glob(in.G),
                                                                  in.gpitch, in.glen, j0, b0, raw, opaque_tid());
     else
-        build_tile<NBITS, BIG, false, BATCH_BCW, BATCH_LOADS, NT>(glob(in.packed), in.nsamps, in.nchans, glob(in.G),
+        build_tile<NBITS, BIG, false, BCW, BATCH_LOADS, NT>(glob(in.packed), in.nsamps, in.nchans, glob(in.G),
                                                                   in.gpitch, in.glen, j0, b0, raw, opaque_tid());
 }
 
-// Stage-1 unit: words [j0, j0 + B_TJ) of the packed row bytes [b0, b0 + BATCH_BCW).
-template <int NT>
+// Stage-1 unit: words [j0, j0 + B_TJ) of the packed row bytes [b0, b0 + BCW).
+template <int NT, int BCW>
 __device__ __forceinline__ void run_build(CInst& in, int64_t j0, int64_t b0, uint8_t* raw) {
     switch (in.nbits * 2 + in.big) {
-        case 2: build_item<1, false, NT>(in, j0, b0, raw); break;
-        case 3: build_item<1, true, NT>(in, j0, b0, raw); break;
-        case 4: build_item<2, false, NT>(in, j0, b0, raw); break;
-        case 5: build_item<2, true, NT>(in, j0, b0, raw); break;
-        case 8: build_item<4, false, NT>(in, j0, b0, raw); break;
-        case 9: build_item<4, true, NT>(in, j0, b0, raw); break;
-        default: build_item<8, false, NT>(in, j0, b0, raw); break;
+        case 2: build_item<1, false, NT, BCW>(in, j0, b0, raw); break;
+        case 3: build_item<1, true, NT, BCW>(in, j0, b0, raw); break;
+        case 4: build_item<2, false, NT, BCW>(in, j0, b0, raw); break;
+        case 5: build_item<2, true, NT, BCW>(in, j0, b0, raw); break;
+        case 8: build_item<4, false, NT, BCW>(in, j0, b0, raw); break;
+        case 9: build_item<4, true, NT, BCW>(in, j0, b0, raw); break;
+        default: build_item<8, false, NT, BCW>(in, j0, b0, raw); break;
     }
 }
 
@@ -183,8 +188,9 @@ struct BlockQueue {
 
 // Thread 0: the next time tile of the current item; or else publish the completed items of
 // exhausted segments, claim the next item (its own XCD's sub-queue first), wait for the
-// segment's dependency once, and decode the item's first unit. nsub: DM sub-tiles per tile.
-__device__ __forceinline__ void next_item(const BArgs* A, BlockQueue* Q, int nsub) {
+// segment's dependency once, and decode the item's first unit. nsub: DM sub-tiles per tile;
+// bcw: packed bytes per row of a stage-1 item.
+__device__ __forceinline__ void next_item(const BArgs* A, BlockQueue* Q, int nsub, int bcw) {
     Q->acquire = 0;
     if (Q->pending && Q->kind == 1 && Q->b + 1 < Q->tt_end) {
         ++Q->b;
@@ -252,7 +258,7 @@ __device__ __forceinline__ void next_item(const BArgs* A, BlockQueue* Q, int nsu
         if (sg.kind == 0) {
             const int64_t nby = in->nby;
             Q->a = unit_at(li / nby, BB_RUN, x) * B_TJ;
-            Q->b = (li % nby) * BATCH_BCW;
+            Q->b = (li % nby) * bcw;
         } else {
             const int64_t per = in->ntiles_dm * nsub;
             const int64_t grp = unit_at(li / per, BT_RUN, x);
@@ -276,7 +282,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(MINW
     static_assert(WAVES * 64 == B_THREADS || WAVES * 64 == 2 * B_THREADS,
                   "stage-1 items take the block's threads (B_THREADS or twice that)");
     constexpr int SWEEP_WORDS = 2 * CC * SW_LW;
-    constexpr int BUILD_WORDS = (build_lds_bytes<1, BATCH_BCW>() + 3) / 4;  // IL = 8 stages the most
+    constexpr int BCW = batch_bcw(CC);
+    constexpr int BUILD_WORDS = (build_lds_bytes<1, BCW>() + 3) / 4;  // IL = 8 stages the most
     __shared__ uint32_t lds[SWEEP_WORDS > BUILD_WORDS ? SWEEP_WORDS : BUILD_WORDS];
     __shared__ BlockQueue Q;
     // Mixed plans: some have few rows in their tiles. Skipping the sums of waves without a row took a
@@ -293,14 +300,14 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(MINW
         Q.skip = 0;
     }
     for (;;) {
-        if (tid == 0) next_item(A, &Q, SW_DT / (K * WAVES));
+        if (tid == 0) next_item(A, &Q, SW_DT / (K * WAVES), BCW);
         __syncthreads();
         if (uni(Q.end)) break;
         if (uni(Q.acquire)) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         if (!uni(Q.skip)) {
             CInst& in = *(CInst*)(A->insts + uni(Q.inst));
             if (uni(Q.kind) == 0) {
-                run_build<WAVES * 64>(in, uni(Q.a), uni(Q.b), reinterpret_cast<uint8_t*>(lds));
+                run_build<WAVES * 64, BCW>(in, uni(Q.a), uni(Q.b), reinterpret_cast<uint8_t*>(lds));
             } else {
                 // Stage-2 unit: sub-tile sub of DM tile dt over time tile tt, the one-plan
                 // kernel's body for the instance's field width (included per case, so that it
@@ -461,6 +468,11 @@ double item_cost(const spp_sweep_plan* p) {
     return static_cast<double>(p->nchans) * (p->nbits <= 2 ? 2.0 : 1.0);
 }
 
+// Stage-1 items side by side in a row of the packed stream.
+int64_t stage1_columns(const spp_batch* b, const spp_sweep_plan* p) {
+    return spp::ceil_div(p->nchans * p->nbits / 8, int64_t(batch_bcw(shape_cc(b->shape))));
+}
+
 // Rounds: every instance's G in one pool when the budget allows, otherwise first-fit
 // decreasing into rounds of half the budget (two pools alternate).
 int plan_rounds(spp_batch* b) {
@@ -546,7 +558,7 @@ QueueTables queue_tables(const spp_batch* b) {
                 const spp_sweep_plan* p = b->plans[t.rinst[s.inst0 + k]];
                 if (kind == 0) {
                     const int64_t ntb = spp::ceil_div(p->gpitch, int64_t(B_TJ));
-                    acc += units_of(ntb, BB_RUN, x) * spp::ceil_div(p->nchans * p->nbits / 8, int64_t(BATCH_BCW));
+                    acc += units_of(ntb, BB_RUN, x) * stage1_columns(b, p);
                 } else {
                     const int64_t ngrp = spp::ceil_div(ntiles_t_of(p), int64_t(b->ntt));
                     acc += units_of(ngrp, BT_RUN, x) * static_cast<int64_t>(p->tile_dm0.size()) * nsub;
@@ -693,7 +705,11 @@ extern "C" int spp_batch_get_info(const spp_batch* b, spp_batch_info* info) {
     info->chans_per_stage = shape_cc(b->shape);
     info->build_items = 0;
     info->sweep_items = 0;
-    for (const BSeg& s : t.segs) (s.kind == 0 ? info->build_items : info->sweep_items) += s.total;
+    for (const BSeg& s : t.segs)
+        if (s.kind == 1) info->sweep_items += s.total;
+    // Stage-1 work in units of B_TJ words x 32 packed bytes for every shape (an item takes one or two).
+    for (const spp_sweep_plan* p : b->plans)
+        info->build_items += spp::ceil_div(p->gpitch, int64_t(B_TJ)) * spp::ceil_div(p->nchans * p->nbits / 8, int64_t(32));
     return SPP_OK;
 }
 
@@ -773,7 +789,7 @@ extern "C" int spp_batch_bind(spp_batch* b, const uint8_t* const* packed, float*
         d.ld = ld[i];
         d.ntiles_dm = nt;
         d.ntiles_t = ntiles_t_of(p);
-        d.nby = spp::ceil_div(p->nchans * p->nbits / 8, int64_t(BATCH_BCW));
+        d.nby = stage1_columns(b, p);
         d.nbits = p->nbits;
         d.big = p->big;
         d.use32 = p->use32 ? 1 : 0;
