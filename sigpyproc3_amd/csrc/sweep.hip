@@ -70,7 +70,10 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 //     channels x 20011, 64 rows: 25 (34 with 16 rows); 2-bit 4096 x 20000, 64 rows: 268 (353); 8-bit
 //     1024 x 40000, 40 rows, 120 blocks: 89 (116). Past 128 some CUs run two: 8-bit 141 blocks 131
 //     against 116, 2-bit 150 blocks 110 against 95;
-//   tiles at most 4/5 full (rows whose delays lie far apart): one row a wave, the waves without a row
+//   4- and 8-bit data of fewer than 128 channels: two rows a wave, which share the few stages' set-up
+//     and stores (72 channels, 37 rows, 4-bit x 851845 67 against 80 with one row a wave, 8-bit x
+//     400000 42 against 46; at 200 4-bit channels 82 / 86, at 336 level);
+//   tiles at most 4/5 full, 3/4 at 4-bit (rows whose delays lie far apart): one row a wave, the waves without a row
 //     skip the sums. 256 rows of 1024 channels x 2^17 in 29 tiles, 1 / 2 / 4 / 8-bit: 389 426 824 1007
 //     (535 553 1114 1320 with sums over padding rows; best other shape at 4-bit 1060); in 52 tiles
 //     545 564 1120 1322 (855 882 1799 2262). At 18 tiles 360 358 698 842 against 350 362 661 802;
@@ -84,7 +87,9 @@ int auto_variant(const spp_sweep_plan* p, int64_t max_len) {
     const int64_t T = (p->nbits <= 2 ? 8 : 4) * SW_S;
     const int64_t blocks = static_cast<int64_t>(p->tile_dm0.size()) * spp::ceil_div(max_len, T);
     if (blocks <= 128) return 6;
-    if (p->ndm * 5 <= static_cast<int64_t>(p->tile_dm0.size()) * SW_DT * 4) return 7;
+    if (p->nbits >= 4 && p->nchans < 128) return p->nbits == 4 ? 3 : 0;
+    const int64_t slots = static_cast<int64_t>(p->tile_dm0.size()) * SW_DT;
+    if (p->nbits == 4 ? p->ndm * 4 <= slots * 3 : p->ndm * 5 <= slots * 4) return 7;
     if (p->nbits <= 2) return 4;
     if (p->nbits == 4) return blocks <= 1024 ? 4 : 3;
     return blocks <= 16384 ? 4 : 0;

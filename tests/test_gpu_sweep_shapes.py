@@ -49,10 +49,11 @@ def test_default_shape(nbits, nchans, ndm, blocks):
 
 @pytest.mark.parametrize("nbits", [1, 2, 4, 8])
 @pytest.mark.parametrize("step,per_tile", [(60, 5), (250, 2), (300, 1), (17, 15), (20, 13)])
-def test_tiles_with_few_rows(nbits, step, per_tile):
+@pytest.mark.parametrize("nchans", [40, 136])
+def test_tiles_with_few_rows(nbits, step, per_tile, nchans):
     # tiles hold the rows within 252 samples; each row ends `step` samples before the last, so whole
     # blocks of some rows lie past their ends
-    ndm, nchans, T = 41, 40, 2048 if nbits <= 2 else 1024
+    ndm, T = 41, 2048 if nbits <= 2 else 1024
     table = np.round(step * np.arange(ndm)[:, None] * np.linspace(0, 1, nchans)[None, :]).astype(np.int32)
     tiles = -(-ndm // per_tile)
     _check(np.random.default_rng(nbits * 1000 + step), table, (128 // tiles + 12) * T + 333, nbits, tiles)
