@@ -348,7 +348,10 @@ int spp_boxcar_mf_noalloc(const float* z, int64_t ldz, int64_t nrows, const int6
  * box sums of one width equal. Rows whose good size is odd take spp_boxcar_mf's FFT path
  * (one row at a time); a row of exactly Ng (odd) samples is refused with SPP_EINVAL.
  * Row lengths 1 <= n <= min(ldx, 2^31 - 1) and n >= the largest width; window >= 1.
- * workspace: spp_normalise_boxcar_mf_workspace_size bytes. Synchronises the stream.
+ * workspace: spp_normalise_boxcar_mf_workspace_size bytes for the same row lengths and widths; one
+ * sized for as many or more rows of at least these lengths serves too (rows with an odd good
+ * size need the space of their own row lengths).
+ * Synchronises the stream.
  */
 int spp_normalise_boxcar_mf_workspace_size(int64_t nrows, const int64_t* row_len_host,
                                            const int32_t* widths_host, int32_t nwidths, int64_t* bytes);

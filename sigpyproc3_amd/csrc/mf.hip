@@ -1298,7 +1298,8 @@ int64_t nb_chunk(int64_t nrows, int64_t max_len) {
     return segs * RN_SEG;
 }
 
-NbLayout nb_layout(int64_t nrows, const int64_t* row_len, const int32_t* widths, int32_t nw) {
+// chb: outputs per block (0: what nb_chunk says).
+NbLayout nb_layout(int64_t nrows, const int64_t* row_len, const int32_t* widths, int32_t nw, int64_t chb = 0) {
     NbLayout l;
     int64_t max_len = 1, sumw = 0;
     for (int64_t i = 0; i < nrows; ++i) {
@@ -1311,7 +1312,7 @@ NbLayout nb_layout(int64_t nrows, const int64_t* row_len, const int32_t* widths,
         }
     }
     for (int i = 0; i < nw; ++i) sumw += widths[i];
-    l.chb = nb_chunk(nrows, max_len);
+    l.chb = chb > 0 ? chb : nb_chunk(nrows, max_len);
     l.nb_row = std::max<int64_t>(1, spp::ceil_div(max_len, l.chb));
     int64_t off = 0;
     l.off_rows = off; off = align256(off + static_cast<int64_t>(sizeof(NbRow)) * nrows);
@@ -1384,7 +1385,10 @@ extern "C" int spp_normalise_boxcar_mf(const float* x, int64_t ldx, int64_t nrow
         rows[i].odd = rows[i].ng & 1;
         if (rows[i].odd) odd_rows.push_back(i);
     }
-    const NbLayout l = nb_layout(nrows, row_len_host, widths_host, nwidths);
+    // Fewer or shorter rows can take more, shorter blocks than the rows a workspace was sized for:
+    // blocks as long as the partials need to fit it (16 segments need no more than any longer call).
+    NbLayout l = nb_layout(nrows, row_len_host, widths_host, nwidths);
+    while (workspace_bytes < l.bytes && l.chb < RN_CHB) l = nb_layout(nrows, row_len_host, widths_host, nwidths, 2 * l.chb);
     SPP_REQUIRE(workspace_bytes >= l.bytes, "workspace too small: %lld < %lld",
                 static_cast<long long>(workspace_bytes), static_cast<long long>(l.bytes));
     const int64_t nblocks = nrows * l.nb_row;
