@@ -564,7 +564,7 @@ extern "C" int spp_subband(const void* in, int nbits, int big, int64_t nchans, i
         SPP_LAUNCHED("k_subband_f32");
         return SPP_OK;
     }
-    if (nbits == 8 && spp::subband8_applies(in, nchans, nout, nsubs))
+    if (nbits == 8 && spp::subband8_applies(in, nchans, nsamps, nout, nsubs))
         return spp::launch_subband8(static_cast<const uint8_t*>(in), delays, chan_to_sub, out, nchans, nsamps, nout,
                                     nsubs, out_size, st);
     return launch_int<1>(static_cast<const uint8_t*>(in), nbits, big, delays, chan_to_sub, out,

@@ -8,7 +8,7 @@
 namespace spp {
 
 // True when the kernel takes this launch (nbits == 8).
-bool subband8_applies(const void* in, int64_t nchans, int64_t nout, int64_t nsubs);
+bool subband8_applies(const void* in, int64_t nchans, int64_t nsamps, int64_t nout, int64_t nsubs);
 
 // out[t * nsubs + chan_to_sub[c]] += in[t + delays[c]][c] over all channels, t < nout, on an `out`
 // that is already zero; flat indices >= out_size are dropped.

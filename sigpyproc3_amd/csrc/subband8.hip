@@ -4,8 +4,9 @@
 // The byte-staged kernel (k_gulp_int) combines channel groups with float atomics, one per
 // (output, band), and runs at the rate the L2 takes those: 2e10 per second. Here a block owns
 // SB_T outputs and every band whose first channel lies in its channel range, so each output is
-// one plain store. That needs bands of consecutive channels (a non-decreasing map): a block
-// reads the whole map once to find out, and keeps the atomics for any other map.
+// one plain store. That needs bands of consecutive channels (a map that only rises or only falls): a
+// block reads the whole map once to find out, and keeps the atomics for any other map and
+// for the bands that are too wide for one block.
 //
 // A stage takes SB_Q groups of 16 channels: SB_Q lanes read 16 bytes each of one row, side by
 // side. A lane loads 4 rows, transposes them in registers (v_perm), and writes 4 consecutive
@@ -17,9 +18,10 @@
 // v_perm; the even ones as the raw 32-bit sum minus 256 times the odd sum).
 //
 // Measured on 1024 channels x 131072 samples, 64 bands, maximum delay 5077 (166 MB in and out):
-// 406 -> 78 us (2.1 TB/s). Of that the loads alone take 48, the sums about 25 (a block has two
-// stages, so half of them overlap no load) and the stores 8. Narrower stages (32 channels, four
-// blocks per CU) run 87, 2048 outputs per block 105.
+// a whole call 407 -> 69 us, 7 of them zeroing the output. The loads alone take 48, the sums about 25
+// (a block has two stages, so half of them overlap no load) and the stores 8. Narrower stages (32
+// channels, four blocks per CU) ran 87 when this form ran 78, 2048 outputs per block 105. (The map
+// is looked through by shuffles: LDS atomics on one address took 4 us more per block.)
 #include "spp_subband8.hpp"
 
 #include "spp_common.hpp"
@@ -35,6 +37,7 @@ constexpr int SB_Q = 4;                    // 16-channel groups per stage
 constexpr int SB_CH = 16 * SB_Q;           // channels per stage
 constexpr int SB_NRB = SB_T / 4 + 1;       // series dwords of a channel: its outputs' and the funnel's upper one
 constexpr int SB_PITCH = SB_NRB + 2;       // a spare dword, and odd: the groups a wave writes fall 16 banks apart
+constexpr int SB_WIDE = 256;               // channels of a band that one block sums at most
 constexpr int SB_UNITS = 6;                // units of the next stage each thread loads ahead
 // Word 3 of a raw buffer resource on gfx9-family GPUs: 32-bit data format, no swizzle.
 constexpr int kBufferFlags = 0x00020000;
@@ -66,7 +69,8 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
     __shared__ uint32_t series[SB_CH * SB_PITCH];
     __shared__ int32_t sdel[2][SB_CH], ssub[2][SB_CH], sshift[2][SB_CH];
     __shared__ int32_t gmin[2][SB_Q], gmax[2][SB_Q];
-    __shared__ int32_t bound[2];
+    __shared__ int4 bound[SB_THREADS / 64];  // per wave: band starts about the block's range
+    __shared__ int32_t order[SB_THREADS / 64];
     // consecutive blocks on one XCD: the channel groups of one time tile share row lines in its L2
     const int64_t logical = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
     if (logical >= nblocks) return;
@@ -77,10 +81,15 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
     const int64_t cb = (logical % ngroups) * chans_per_group;
     const int64_t ce = min(nchans, cb + chans_per_group);
 
-    // Bands of consecutive channels? Then this block's channels are the bands that start in
-    // [cb, ce): from the first band start at or after cb to the first at or after ce.
-    bool sorted = true;
-    int first = INT_MAX, last = INT_MAX;
+    // Bands of consecutive channels (a non-decreasing or non-increasing map)? Then this block's
+    // channels are the bands that start in [cb, ce), to their ends. A band of more than SB_WIDE
+    // channels is not one block's chain of stages: the blocks whose ranges it covers each add
+    // their part of it. 1024 channels x 131072, one band of 961 among 63 of one channel: 197 us in
+    // one block, 175 shared; 4096 x 16384, one of 3969 among 127: 463 and 90; four of 200: 114, and
+    // 152 if bands of more than 128 are shared.
+    bool valid = true, up = true, down = true;
+    int start_cb = 0, after_cb = static_cast<int>(nchans);  // band starts: last up to cb, first past it
+    int start_ce = 0, after_ce = static_cast<int>(nchans);  // and about ce
     for (int64_t c4 = tid; c4 < nchans; c4 += 4 * SB_THREADS) {
         int s[4], prev[4];
 #pragma unroll
@@ -91,21 +100,50 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int64_t c = min(c4 + j * SB_THREADS, nchans - 1);
-            sorted = sorted && s[j] >= max(prev[j], 0) && s[j] < nsubs;
-            if (s[j] != prev[j] || c == 0) {
-                if (c >= ce) last = min(last, static_cast<int>(c));
-                else if (c >= cb) first = min(first, static_cast<int>(c));
+            const int c = static_cast<int>(min(c4 + j * SB_THREADS, nchans - 1));
+            valid = valid && s[j] >= 0 && s[j] < nsubs;
+            up = up && s[j] >= prev[j];
+            down = down && s[j] <= prev[j];
+            if (s[j] != prev[j]) {
+                if (c <= cb) start_cb = max(start_cb, c);
+                else after_cb = min(after_cb, c);
+                if (c <= ce) start_ce = max(start_ce, c);
+                else after_ce = min(after_ce, c);
             }
         }
     }
-    if (tid < 2) bound[tid] = static_cast<int>(nchans);
-    sorted = __syncthreads_and(sorted);
-    atomicMin(&bound[0], first);
-    atomicMin(&bound[1], last);
+    up = __all(valid && up);
+    down = __all(valid && down);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        start_cb = max(start_cb, __shfl_xor(start_cb, o));
+        after_cb = min(after_cb, __shfl_xor(after_cb, o));
+        start_ce = max(start_ce, __shfl_xor(start_ce, o));
+        after_ce = min(after_ce, __shfl_xor(after_ce, o));
+    }
+    if (lane == 0) {
+        bound[tid >> 6] = make_int4(start_cb, after_cb, start_ce, after_ce);
+        order[tid >> 6] = (up ? 1 : 0) | (down ? 2 : 0);
+    }
     __syncthreads();
-    const int64_t lo = sorted ? min<int64_t>(bound[0], ce) : cb;
-    const int64_t hi = sorted ? (lo < ce ? bound[1] : ce) : ce;
+    int4 bd = bound[0];
+    int ord = order[0];
+#pragma unroll
+    for (int w = 1; w < SB_THREADS / 64; ++w) {
+        const int4 b = bound[w];
+        bd = make_int4(max(bd.x, b.x), min(bd.y, b.y), max(bd.z, b.z), min(bd.w, b.w));
+        ord &= order[w];
+    }
+    const bool sorted = __builtin_amdgcn_readfirstlane(ord) != 0;
+    const int head0 = __builtin_amdgcn_readfirstlane(bd.x), head1 = __builtin_amdgcn_readfirstlane(bd.y);
+    const int tail0 = __builtin_amdgcn_readfirstlane(bd.z), tail1 = __builtin_amdgcn_readfirstlane(bd.w);
+    const bool head = sorted && head0 < cb;                // the block's first channel is in a band before it,
+    const bool tail = sorted && ce < nchans && tail0 < ce;  // its last one in a band that goes on
+    bool shared_head = head && head1 - head0 > SB_WIDE;
+    const bool shared_tail = tail && tail1 - tail0 > SB_WIDE;
+    const int64_t lo = head && !shared_head ? head1 : cb;
+    const int64_t hi = tail && !shared_tail ? tail1 : ce;
+    if (lo >= ce) return;  // one band of another block
 
     uint32_t raw = 0, odd = 0, wide[4] = {0, 0, 0, 0};
     int packed = 0;  // channels in the 16-bit lanes
@@ -127,8 +165,9 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
     const int64_t room = out_size - ta * nsubs;  // floats from orow on that may be written
     f32x4_any held[4];                           // [output][band]
     int nheld = 0, held0 = 0;
+    bool held_whole = sorted;  // the held bands are this block's alone: plain stores
     auto drain = [&]() {
-        if (nheld == 4 && sorted && room >= 3 * nsubs + held0 + 4) {
+        if (nheld == 4 && held_whole && room >= 3 * nsubs + held0 + 4) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 if (j < nvalid) *reinterpret_cast<f32x4_any*>(orow + j * nsubs + held0) = held[j];
@@ -140,7 +179,7 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
                     const int64_t i = j * nsubs + held0 + b;
                     if (j < nvalid && i < room) {
                         const float v = b == 0 ? held[j][0] : b == 1 ? held[j][1] : b == 2 ? held[j][2] : held[j][3];
-                        if (sorted) orow[i] = v;
+                        if (held_whole) orow[i] = v;
                         else atomicAdd(orow + i, v);
                     }
                 }
@@ -148,11 +187,14 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
         }
         nheld = 0;
     };
-    auto flush = [&](int band) {
+    auto flush = [&](int band, bool whole) {
         widen();
         if (band >= 0) {
-            if (nheld == 4 || (nheld > 0 && band != held0 + nheld)) drain();
-            if (nheld == 0) held0 = band;
+            if (nheld == 4 || (nheld > 0 && (band != held0 + nheld || whole != held_whole))) drain();
+            if (nheld == 0) {
+                held0 = band;
+                held_whole = whole;
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float v = static_cast<float>(wide[j]);
@@ -346,7 +388,11 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
                     odd += odd_bytes(vj);
                     ++packed;
                 }
-                if ((end4 >> j) & 1u) flush(__builtin_amdgcn_readlane(my_sub, k + j));
+                if ((end4 >> j) & 1u) {
+                    flush(__builtin_amdgcn_readlane(my_sub, k + j),
+                          sorted && !shared_head && !(shared_tail && c + k + j + 1 >= hi));
+                    shared_head = false;
+                }
             }
             if (packed > 252) widen();  // 257 samples of 255 fit a 16-bit lane
         }
@@ -359,17 +405,24 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
 
 namespace spp {
 
-bool subband8_applies(const void* in, int64_t nchans, int64_t nout, int64_t nsubs) {
-    // Rows of whole dwords; exact float sums for maps that fall back to atomics.
+bool subband8_applies(const void* in, int64_t nchans, int64_t nsamps, int64_t nout, int64_t nsubs) {
+    // Rows of whole dwords; exact float sums for the atomics.
     if (nchans % 4 != 0 || reinterpret_cast<uintptr_t>(in) % 4 != 0 || nchans * 255 >= (int64_t(1) << 24)) return false;
-    // The byte-staged kernel pays an atomic per output and band, this one a block's chain of
-    // stages per band. Measured, this one against that (us): 64-channel bands 75 / 143 (16 of
-    // 1024 channels x 131072), 17-channel 298 / 1334 (128 of 2176 x 174534); 128-channel 128 / 149
-    // (32 of 4096 x 65536) but 110 / 98 with only 8 bands; 512-channel 292 / 112. Below about
-    // 2e5 outputs a single block's latency shows: 27 / 11 (8 of 72 x 16384), 23 / 30 (8 of
-    // 512 x 32768).
+    // The byte-staged kernel pays an atomic per output and band (or channel group, of which a short
+    // gulp gets more than bands), this one a block's chain of stages per band. Measured, this one
+    // against that (us): 64-channel bands 63 / 143 (16 of 1024 channels x 131072), 17-channel 298 /
+    // 1334 (128 of 2176 x 174534); 128-channel 116 / 152 (32 of 4096 x 65536) but 110 / 98 with
+    // only 8 bands; 512-channel 292 / 112. A map that is not sorted costs both the same atomics.
     const int64_t width = ceil_div(nchans, nsubs);
-    return nout * nsubs >= 200000 && (width <= 64 || (width <= 128 && nsubs >= 32));
+    if (width > 64 && (width > 128 || nsubs < 32)) return false;
+    // A block loads its 16-channel groups' rows over their whole delay spread, however few of them a
+    // channel keeps, so the atomics must pay for the spread as well as for a block's latency. Without
+    // spread, 8 bands x 32768 outputs: 23 / 12.5 (64 channels), 22.5 / 33 (512 channels, 32 groups);
+    // 16 x 32768 25 / 31. With 8192 rows of spread: 8 x 98304 82 / 51, 32 x 98304 97 / 162, 8 x 458752
+    // 117 / 236; with 16384: 8 x 131072 (32 channels) 105 / 46, 8 x 491520 119 / 121.
+    const int64_t groups = std::min(ceil_div(int64_t(8) * device_cu_count(), ceil_div(nout, int64_t(512))), ceil_div(nchans, int64_t(16)));
+    const int64_t spread = (nsamps - nout) * 16 / std::max<int64_t>(nchans, 16);
+    return nout * std::max(nsubs, groups) >= 300000 + 110 * spread;
 }
 
 int launch_subband8(const uint8_t* in, const int32_t* delays, const int32_t* chan_to_sub, float* out, int64_t nchans,
