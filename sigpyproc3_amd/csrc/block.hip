@@ -80,7 +80,9 @@ __global__ __launch_bounds__(RB_THREADS) void k_roll_rows4(const float* __restri
 // Measured on 1024 channels x 8192 samples, 512 DM rows: 2436 -> 618 us (4.3e9 adds; the LDS
 // reads alone take 220 at 128 bytes per clock and CU, the rest is the wait of each 5-channel
 // stage). Windows of 128 spare samples and 8 channels run 528 there but leave 2000 channels x
-// 16384, 128 rows (offsets up to 450 apart) to memory: 3670 us against 1697.
+// 16384, 128 rows (offsets up to 450 apart) to memory. Channels added from memory have a stage's 32
+// loads in flight: 1024 x 65536, 32 rows spread over 30000 samples, 1042 us (1587 with a thread per
+// output and one load in flight).
 constexpr int DT_D = 8;         // DM rows per block
 constexpr int DT_K = 4;         // samples per thread
 constexpr int DT_CC = 5;        // channels per stage
@@ -125,7 +127,7 @@ __global__ __launch_bounds__(RB_THREADS) void k_dmt(const float* __restrict__ in
         col = col >= ncols ? col - ncols : col;
         col += mn;
         col = col < 0 ? col + ncols : col;
-        wstart[slot] = mx - mn <= DT_SPREAD && W <= ncols ? col : -1;
+        wstart[slot] = mx - mn <= DT_SPREAD ? col : -1;  // W <= ncols (dmt_in_tiles)
         auto pair = [&](int r) {
             return static_cast<uint32_t>((rel[r] - mn) & 0xffff) | static_cast<uint32_t>(rel[r + 1] - mn) << 16;
         };
@@ -174,18 +176,25 @@ __global__ __launch_bounds__(RB_THREADS) void k_dmt(const float* __restrict__ in
 #pragma unroll
             for (int j = 0; j < K; ++j) acc[r][j] = acc[r][j] + v[r][j];
     };
+    int td[K];  // the thread's samples; those past the last output repeat it
+#pragma unroll
+    for (int j = 0; j < K; ++j) td[j] = min(t0 + tid + RB_THREADS * j, out_cols - 1);
     auto add_direct = [&](int64_t c) {
         const float* __restrict__ row = in + c * ncols;
+        float v[DT_D][K];
 #pragma unroll
         for (int r = 0; r < DT_D; ++r) {
             const int o = static_cast<int>(off[min<int64_t>(i0 + r, ndm - 1) * nchans + c]);
 #pragma unroll
             for (int j = 0; j < K; ++j) {
-                int col = o + t0 + tid + RB_THREADS * j;
-                while (col >= ncols) col -= ncols;
-                acc[r][j] = acc[r][j] + row[col];
+                const int col = o + td[j];
+                v[r][j] = row[col >= ncols ? col - ncols : col];
             }
         }
+#pragma unroll
+        for (int r = 0; r < DT_D; ++r)
+#pragma unroll
+            for (int j = 0; j < K; ++j) acc[r][j] = acc[r][j] + v[r][j];
     };
     for (int64_t c0 = 0; c0 < nchans; c0 += DT_PLAN) {
         bool mine = true;
@@ -294,6 +303,23 @@ extern "C" int spp_roll_rows(const float* in, int64_t nrows, int64_t ncols, cons
     return SPP_OK;
 }
 
+namespace spp {
+
+// True when the tiled transform (k_dmt) takes the call.
+bool dmt_in_tiles(int64_t ncols, int64_t ndm, int64_t out_cols) {
+    // A window must fit the row (with every channel added from memory, 1024 channels x 1024 samples,
+    // 2048 rows take 917 us in tiles and 481 with a thread per output; 1500 samples 1217 and 721), its
+    // byte offsets 32 bits, and a tile must hold four rows or more (it sums eight whatever it holds:
+    // 256 x 300000, offsets far apart, 2 rows 315 and 100, 4 rows 327 and 195; near each other 3
+    // rows 150 and 118, 4 rows 170 and 190). And a tile per CU: 256 rows of 1024 channels x 2048 samples
+    // (64 tiles): 151 us with a thread per output, 402 in small tiles; 512 rows of 336 x 5001 (320
+    // tiles): 203 tiled, 453 with a thread per output.
+    const int64_t by = ceil_div(ndm, int64_t(DT_D)), bx = ceil_div(out_cols, int64_t(RB_THREADS) * DT_K);
+    return ncols >= RB_THREADS * DT_K + DT_SPREAD && ncols < (int64_t(1) << 29) && ndm >= DT_D / 2 && bx * by >= device_cu_count();
+}
+
+}  // namespace spp
+
 extern "C" int spp_dmt(const float* in, int64_t nchans, int64_t ncols, const int64_t* off_host,
                        const int64_t* off, int64_t ndm, int64_t out_cols, float* out, void* stream) {
     spp::clear_error();
@@ -308,10 +334,7 @@ extern "C" int spp_dmt(const float* in, int64_t nchans, int64_t ncols, const int
                         static_cast<long long>(off_host[k]), static_cast<long long>(out_cols));
     }
     const int64_t by = spp::ceil_div(ndm, int64_t(DT_D)), bx = spp::ceil_div(out_cols, int64_t(RB_THREADS) * DT_K);
-    // The tiled form needs a block per CU and 32-bit byte offsets into a row. 256 rows of 1024
-    // channels x 2048 samples (64 tiles): 151 us with a thread per output, 402 in small tiles; 512
-    // rows of 336 x 5001 (320 tiles): 203 tiled, 453 with a thread per output.
-    if (ncols >= (int64_t(1) << 29) || bx * by < spp::device_cu_count()) {
+    if (!spp::dmt_in_tiles(ncols, ndm, out_cols)) {
         const int64_t bx1 = spp::ceil_div(out_cols, int64_t(RB_THREADS));
         SPP_REQUIRE(bx1 <= 0x7fffffffLL, "too many columns");
         hipLaunchKernelGGL(k_dmt_rows, dim3(static_cast<unsigned>(bx1), static_cast<unsigned>(ndm)), dim3(RB_THREADS), 0,
