@@ -22,6 +22,7 @@
 #include "spp_unpack.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -286,12 +287,15 @@ __global__ __launch_bounds__(DD_THREADS) void k_gulp_int(
     }
 }
 
-// Subbands of float32 samples: each band's run of channels summed in order in float32
-// (kernels.py:397-401 adds into the float32 output).
-__global__ __launch_bounds__(DD_THREADS) void k_subband_f32(
+// float32 samples, channels summed in order: float64 for dedisperse (kernels.py:357-361
+// accumulates in float64), float32 for subband (kernels.py:397-401 adds into the float32
+// output); MODE as above. Dedispersion of short gulps takes gulp_f32.hip's small blocks instead
+// (ded_f32_small_blocks says which).
+template <int MODE>
+__global__ __launch_bounds__(DD_THREADS) void k_gulp_f32(
     const float* __restrict__ in, const int32_t* __restrict__ delays,
     const int32_t* __restrict__ chan_to_sub, float* __restrict__ out, int64_t nchans, int64_t nsamps,
-    int64_t nout, int64_t nsubs, int64_t out_size) {
+    int64_t nout, int64_t out_start, int64_t nsubs, int64_t out_size) {
     __shared__ float tile[DDF_ROWS * DDF_STRIDE];
     __shared__ int32_t sdel[DDF_CC];
     __shared__ int32_t ssub[DDF_CC];
@@ -301,14 +305,15 @@ __global__ __launch_bounds__(DD_THREADS) void k_subband_f32(
     const int64_t t0 = static_cast<int64_t>(blockIdx.x) * DD_T;
     const int64_t ta = t0 + tid;
     const int64_t tb = t0 + DD_THREADS + tid;
-    float acc0 = 0, acc1 = 0;
+    using acc_t = std::conditional_t<MODE == 0, double, float>;
+    acc_t acc0 = 0, acc1 = 0;
     int cur_sub = -1;
 
     auto flush_sub = [&](int sub) {
         if (sub >= 0) {
             const int64_t ia = ta * nsubs + sub, ib = tb * nsubs + sub;
-            if (ta < nout && ia < out_size) atomicAdd(out + ia, acc0);
-            if (tb < nout && ib < out_size) atomicAdd(out + ib, acc1);
+            if (ta < nout && ia < out_size) atomicAdd(out + ia, static_cast<float>(acc0));
+            if (tb < nout && ib < out_size) atomicAdd(out + ib, static_cast<float>(acc1));
         }
         acc0 = 0;
         acc1 = 0;
@@ -319,7 +324,7 @@ __global__ __launch_bounds__(DD_THREADS) void k_subband_f32(
         __syncthreads();
         if (tid < ncand) {
             sdel[tid] = delays[c + tid];
-            ssub[tid] = chan_to_sub[c + tid];
+            if constexpr (MODE == 1) ssub[tid] = chan_to_sub[c + tid];
         }
         __syncthreads();
         int dmin, dmax;
@@ -337,18 +342,25 @@ __global__ __launch_bounds__(DD_THREADS) void k_subband_f32(
         }
         __syncthreads();
         for (int k = 0; k < n; ++k) {
-            const int sub = ssub[k];
-            if (sub != cur_sub) {
-                flush_sub(cur_sub);
-                cur_sub = sub;
+            if constexpr (MODE == 1) {
+                const int sub = ssub[k];
+                if (sub != cur_sub) {
+                    flush_sub(cur_sub);
+                    cur_sub = sub;
+                }
             }
             const int rel = sdel[k] - dmin;
-            acc0 += tile[(tid + rel) * DDF_STRIDE + k];
-            acc1 += tile[(tid + DD_THREADS + rel) * DDF_STRIDE + k];
+            acc0 += static_cast<acc_t>(tile[(tid + rel) * DDF_STRIDE + k]);
+            acc1 += static_cast<acc_t>(tile[(tid + DD_THREADS + rel) * DDF_STRIDE + k]);
         }
         c += n;
     }
-    flush_sub(cur_sub);
+    if constexpr (MODE == 1) {
+        flush_sub(cur_sub);
+    } else {
+        if (ta < nout) out[out_start + ta] = static_cast<float>(acc0);
+        if (tb < nout) out[out_start + tb] = static_cast<float>(acc1);
+    }
 }
 
 __global__ void k_fill_f32(float* __restrict__ p, int64_t n, float v) {
@@ -535,8 +547,17 @@ extern "C" int spp_dedisperse(const void* in, int nbits, int big, int64_t nchans
     hipStream_t st = spp::as_stream(stream);
     const int64_t nout = nsamps - max_delay;
     if (nout <= 0) return SPP_OK;  // the reference loop body never runs
-    if (nbits == 32)
-        return spp::launch_ded_f32(static_cast<const float*>(in), delays, out + out_start, nchans, nsamps, nout, st);
+    if (nbits == 32) {
+        if (spp::ded_f32_small_blocks(nchans, nout, max_delay))
+            return spp::launch_ded_f32(static_cast<const float*>(in), delays, out + out_start, nchans, nsamps, nout, st);
+        const int64_t bx = spp::ceil_div(nout, DD_T);
+        SPP_REQUIRE(bx <= 0x7fffffffLL, "gulp too long");
+        hipLaunchKernelGGL((k_gulp_f32<0>), dim3(static_cast<unsigned>(bx)), dim3(DD_THREADS), 0, st,
+                           static_cast<const float*>(in), delays, nullptr, out, nchans, nsamps, nout,
+                           out_start, int64_t(0), int64_t(0));
+        SPP_LAUNCHED("k_gulp_f32");
+        return SPP_OK;
+    }
     return launch_int<0>(static_cast<const uint8_t*>(in), nbits, big, delays, nullptr, out, nchans,
                          nsamps, nout, out_start, 0, 0, st);
 }
@@ -558,10 +579,10 @@ extern "C" int spp_subband(const void* in, int nbits, int big, int64_t nchans, i
     if (rc) return rc;
     if (nbits == 32) {
         const int64_t bx = spp::ceil_div(nout, DD_T);
-        hipLaunchKernelGGL(k_subband_f32, dim3(static_cast<unsigned>(bx)), dim3(DD_THREADS), 0, st,
+        hipLaunchKernelGGL((k_gulp_f32<1>), dim3(static_cast<unsigned>(bx)), dim3(DD_THREADS), 0, st,
                            static_cast<const float*>(in), delays, chan_to_sub, out, nchans, nsamps,
-                           nout, nsubs, out_size);
-        SPP_LAUNCHED("k_subband_f32");
+                           nout, int64_t(0), nsubs, out_size);
+        SPP_LAUNCHED("k_gulp_f32");
         return SPP_OK;
     }
     if (nbits == 8 && spp::subband8_applies(in, nchans, nsamps, nout, nsubs))

@@ -19,6 +19,7 @@
 
 #include "spp_common.hpp"
 
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -238,6 +239,26 @@ __global__ __launch_bounds__(64 * FC_WAVES) void k_ded_f32(const float* __restri
 }  // namespace
 
 namespace spp {
+
+bool ded_f32_small_blocks(int64_t nchans, int64_t nout, int64_t max_delay) {
+    // The 512-output blocks read half as much around their windows and sum up to 256 rows of delay
+    // spread in one pass of 16 channels; this kernel's 64-output blocks fill the chip eight times
+    // sooner and load passes ahead, but a pass spans 96 rows. So: passes of either kind (the mean
+    // number of channels that fit one), times what a pass takes (us, measured over 1 to 1024 channels
+    // x 16384 to 1000000 samples, per block on each CU). This kernel against the other: 1024 x 16384
+    // 40 / 659, 256 x 131072 at a delay of 5000 221 / 300, 64 x 524288 at 32000 970 / 1440, but
+    // 8 x 131072 14 / 8, 3 x 262144 45 / 21, 64 x 262144 at 1024 103 / 79, 512 x 393216 at 8192
+    // 1024 / 810.
+    auto passes = [&](int64_t spread, int64_t width) {
+        const int64_t fit = max_delay > 0 ? std::min(width, 1 + spread * nchans / max_delay) : width;
+        return static_cast<double>(ceil_div(nchans, fit));
+    };
+    const double cus = device_cu_count();
+    const double here = passes(FC_SPREAD, FC_CC), blocks = ceil_div(nout, int64_t(FC_T)) / cus;
+    const double there = passes(256, 16), blocks512 = ceil_div(nout, int64_t(512)) / cus;
+    const double chain = nchans <= 16 ? 7.0 : 11.0;  // a pass of the other on an idle chip
+    return std::max(6.0 + here, blocks * (1.6 + 0.4 * here)) <= 1.05 * there * std::max(chain, 5.0 * blocks512);
+}
 
 int launch_ded_f32(const float* in, const int32_t* delays, float* out, int64_t nchans, int64_t nsamps, int64_t nout,
                    hipStream_t st) {
