@@ -430,9 +430,10 @@ template <int MODE>
 int launch_int(const uint8_t* in, int nbits, int big, const int32_t* delays, const int32_t* cts,
                float* out, int64_t nchans, int64_t nsamps, int64_t nout, int64_t out_start,
                int64_t nsubs, int64_t out_size, hipStream_t st) {
-    if (MODE == 0 && spp::gulp_swar_applies(nbits, nchans))
-        return launch_swar(in, nbits, big, delays, out, nchans, nsamps, nout, out_start, st);
     const int64_t row_bytes = nchans * nbits / 8;
+    const bool wide = row_bytes % 4 == 0 && reinterpret_cast<uintptr_t>(in) % 4 == 0;
+    if (MODE == 0 && spp::gulp_swar_applies(nbits, wide, nchans, nout, nsamps - nout))
+        return launch_swar(in, nbits, big, delays, out, nchans, nsamps, nout, out_start, st);
     const int64_t bx = spp::ceil_div(nout, DD_T);
     SPP_REQUIRE(bx <= 0x7fffffffLL, "gulp too long");
     // Split channels across blocks until the grid fills the device (integer sums are exact, so
@@ -486,7 +487,6 @@ int launch_int(const uint8_t* in, int nbits, int big, const int32_t* delays, con
     const int64_t nblocks = bx * groups;
     SPP_REQUIRE(nblocks <= 0x7ffffff0LL, "gulp too long");
     dim3 grid(static_cast<unsigned>(spp::ceil_div(nblocks, int64_t(8)) * 8));
-    const bool wide = row_bytes % 4 == 0 && reinterpret_cast<uintptr_t>(in) % 4 == 0;
     const bool narrow = cpg <= 16;
     // 64-channel tiles of DD_ROWS_LOW rows (4 blocks per CU instead of 3) when twice the mean
     // delay spread across DD_CC channels fits them; wider spreads split into more stages there.

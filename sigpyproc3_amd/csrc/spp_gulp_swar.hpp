@@ -12,8 +12,9 @@ namespace spp {
 // or wide stages.
 enum class GulpForm { normal, compact, wide };
 
-// True when the SWAR kernel takes this launch: 1/2/4/8-bit rows of at least 4 bytes.
-bool gulp_swar_applies(int nbits, int64_t nchans);
+// True when the SWAR kernel takes this launch: 1/2/4/8-bit rows of at least 4 bytes, in gulps long
+// enough for it where 1/2-bit rows are not aligned (whole dwords on a 4-byte aligned stream).
+bool gulp_swar_applies(int nbits, bool aligned, int64_t nchans, int64_t nout, int64_t max_delay);
 
 // out[out_start + t] (t < nout) = sum over channels of x[t + delays[c]][c], with x[row] for
 // row < 0 taken from row + nsamps and rows >= nsamps read as 0 (only outputs t >= nout reach
