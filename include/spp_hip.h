@@ -102,9 +102,9 @@ int spp_sweep_plan_destroy(spp_sweep_plan* plan);
 /* Block shapes of the stage-2 kernel (DM rows per wave x waves x channels per stage):
  * 1/2-bit data: 0 = 2x8x16, 1 = 2x8x20, 2 = 2x8x8 (6 waves per SIMD), 3 = 2x8x12 (6 waves per
  *               SIMD), 4 = 1x16x16 (8 waves per SIMD), 5 = 1x16x12 (8 waves per SIMD),
- *               6 = 1x8x32 (blocks of 8 rows), 7 = 4 for tiles with few rows;
+ *               6 = 1x8x32 (blocks of 8 rows), 7 = 4 for tiles with few rows, 8 = 1x8x16;
  * 4/8-bit data: 0 = 2x8x12 (6 waves per SIMD), 1 = 2x8x16, 2 = 4x4x8, 3 = 2x8x8,
- *               4 = 1x16x16, 5 = 1x16x12 (8 waves per SIMD), 6 = 1x8x16 (4-bit) or 1x8x32,
+ *               4 = 1x16x16, 5 = 1x16x12 (8 waves per SIMD), 6 and 8 = 1x8x16,
  *               7 = 4 for tiles with few rows.
  * All give identical results. Each execution takes the shape that suits its size unless
  * spp_sweep_plan_set_variant has picked one for the plan (the autotuner times them). */

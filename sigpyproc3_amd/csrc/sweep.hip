@@ -65,11 +65,15 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
 // The block shape of an execution whose longest row has max_len samples (launch_sweep lists them),
 // by its count of 16-row blocks. Measured (us of k_sweep):
-//   <= 128 blocks: half the CUs or more would hold no 16-row block, so blocks of 8 rows; one fits a
-//     CU, so it may take 128 KB of LDS, and 32 channels a stage halve the barriers. 1-bit 336
+//   <= 128 blocks: half the CUs or more would hold no 16-row block, so blocks of 8 rows. 1-bit 336
 //     channels x 20011, 64 rows: 25 (34 with 16 rows); 2-bit 4096 x 20000, 64 rows: 268 (353); 8-bit
 //     1024 x 40000, 40 rows, 120 blocks: 89 (116). Past 128 some CUs run two: 8-bit 141 blocks 131
-//     against 116, 2-bit 150 blocks 110 against 95;
+//     against 116, 2-bit 150 blocks 110 against 95. 1/2-bit data take 32 channels a stage up to 64
+//     blocks (half the barriers: 2-bit 1024 x 20000, 40 blocks, 90 a whole call against 99 with 16); their
+//     128 KB of LDS keep a CU's other streams out, and past 64 blocks that costs more than it
+//     gives: four streams of 2-bit 256 x 32768, 128 rows, 128 blocks take 28 a call with 32 channels, 23 with
+//     16 (alone 32 and 34); 4/8-bit data gain nothing alone (8-bit 1024 x 40000: 124 either way)
+//     and four streams take 137 and 113, so 16 throughout;
 //   4- and 8-bit data of fewer than 128 channels: two rows a wave, which share the few stages' set-up
 //     and stores (72 channels, 37 rows, 4-bit x 851845 67 against 80 with one row a wave, 8-bit x
 //     400000 42 against 46; at 200 4-bit channels 82 / 86, at 336 level);
@@ -86,7 +90,7 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 int auto_variant(const spp_sweep_plan* p, int64_t max_len) {
     const int64_t T = (p->nbits <= 2 ? 8 : 4) * SW_S;
     const int64_t blocks = static_cast<int64_t>(p->tile_dm0.size()) * spp::ceil_div(max_len, T);
-    if (blocks <= 128) return 6;
+    if (blocks <= 128) return p->nbits <= 2 && blocks > 64 ? 8 : 6;
     if (p->nbits >= 4 && p->nchans < 128) return p->nbits == 4 ? 3 : 0;
     const int64_t slots = static_cast<int64_t>(p->tile_dm0.size()) * SW_DT;
     if (p->nbits == 4 ? p->ndm * 4 <= slots * 3 : p->ndm * 5 <= slots * 4) return 7;
@@ -199,7 +203,7 @@ extern "C" int spp_sweep_plan_create(const int32_t* table_host, int64_t ndm, int
     return SPP_OK;
 }
 
-extern "C" int spp_sweep_variant_count(void) { return 8; }
+extern "C" int spp_sweep_variant_count(void) { return 9; }
 
 extern "C" int spp_sweep_plan_set_variant(spp_sweep_plan* p, int variant) {
     spp::clear_error();
@@ -340,6 +344,7 @@ int launch_sweep(const spp_sweep_plan* p, const Extent& e, char* ws, float* plan
             case 5: return launch_sweep_v<NBITS, USE32, 1, 16, 12, 8>(p, e, ws, plane, ld, st);
             case 7: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8, true>(p, e, ws, plane, ld, st);
             case 6: return launch_sweep_v<NBITS, USE32, 1, 8, 32, 2>(p, e, ws, plane, ld, st);
+            case 8: return launch_sweep_v<NBITS, USE32, 1, 8, 16, 4>(p, e, ws, plane, ld, st);
             default: return launch_sweep_v<NBITS, USE32, 2, 8, 16, 4>(p, e, ws, plane, ld, st);
         }
     } else {
@@ -350,7 +355,8 @@ int launch_sweep(const spp_sweep_plan* p, const Extent& e, char* ws, float* plan
             case 4: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8>(p, e, ws, plane, ld, st);
             case 5: return launch_sweep_v<NBITS, USE32, 1, 16, 12, 8>(p, e, ws, plane, ld, st);
             case 7: return launch_sweep_v<NBITS, USE32, 1, 16, 16, 8, true>(p, e, ws, plane, ld, st);
-            case 6: return launch_sweep_v<NBITS, USE32, 1, 8, (NBITS == 4 ? 16 : 32), 2>(p, e, ws, plane, ld, st);
+            case 6:
+            case 8: return launch_sweep_v<NBITS, USE32, 1, 8, 16, 4>(p, e, ws, plane, ld, st);
             default: return launch_sweep_v<NBITS, USE32, 2, 8, 12, 6>(p, e, ws, plane, ld, st);
         }
     }
