@@ -74,9 +74,12 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 //     gives: four streams of 2-bit 256 x 32768, 128 rows, 128 blocks take 28 a call with 32 channels, 23 with
 //     16 (alone 32 and 34); 4/8-bit data gain nothing alone (8-bit 1024 x 40000: 124 either way)
 //     and four streams take 137 and 113, so 16 throughout;
-//   4- and 8-bit data of fewer than 128 channels: two rows a wave, which share the few stages' set-up
-//     and stores (72 channels, 37 rows, 4-bit x 851845 67 against 80 with one row a wave, 8-bit x
-//     400000 42 against 46; at 200 4-bit channels 82 / 86, at 336 level);
+//   4- and 8-bit data of fewer than 128 channels in tiles more than half full: two rows a wave,
+//     which share the few stages' set-up and stores (72 channels, 37 rows, 4-bit x 851845 67 against
+//     80 with one row a wave, 8-bit x 400000 42 against 46; at 200 4-bit channels 82 / 86, at 336
+//     level). Emptier tiles take the next line's shape: 48 rows of 100 8-bit channels x 262144 in
+//     6 / 12 / 48 tiles 49 73 243 (two rows a wave 65 120 442), of 72 4-bit ones x 400000 55 82 275
+//     (59 102 367);
 //   tiles at most 4/5 full, 3/4 at 4-bit (rows whose delays lie far apart): one row a wave, the waves without a row
 //     skip the sums. 256 rows of 1024 channels x 2^17 in 29 tiles, 1 / 2 / 4 / 8-bit: 389 426 824 1007
 //     (535 553 1114 1320 with sums over padding rows; best other shape at 4-bit 1060); in 52 tiles
@@ -91,8 +94,8 @@ int auto_variant(const spp_sweep_plan* p, int64_t max_len) {
     const int64_t T = (p->nbits <= 2 ? 8 : 4) * SW_S;
     const int64_t blocks = static_cast<int64_t>(p->tile_dm0.size()) * spp::ceil_div(max_len, T);
     if (blocks <= 128) return p->nbits <= 2 && blocks > 64 ? 8 : 6;
-    if (p->nbits >= 4 && p->nchans < 128) return p->nbits == 4 ? 3 : 0;
     const int64_t slots = static_cast<int64_t>(p->tile_dm0.size()) * SW_DT;
+    if (p->nbits >= 4 && p->nchans < 128 && p->ndm * 2 > slots) return p->nbits == 4 ? 3 : 0;
     if (p->nbits == 4 ? p->ndm * 4 <= slots * 3 : p->ndm * 5 <= slots * 4) return 7;
     if (p->nbits <= 2) return 4;
     if (p->nbits == 4) return blocks <= 1024 ? 4 : 3;

@@ -63,6 +63,13 @@ def test_8bit_shapes():
     assert [_shape(8, 128, n, 200) for n in (13, 12)] == [4, 7]
 
 
+@pytest.mark.parametrize(("nbits", "full"), [(4, 3), (8, 0)])
+def test_narrow_bands_in_sparse_tiles(nbits, full):
+    # fewer than 128 channels: two rows a wave only in tiles more than half full
+    assert [_shape(nbits, 126, n, 200) for n in (16, 9, 8, 1)] == [full, full, 7, 7]
+    assert [_shape(nbits, 126, 64, 64 // per * 20, per) for per in (8, 4, 2, 1)] == [7, 7, 7, 7]
+
+
 def test_a_shape_that_was_set_stays():
     lib = _lib.load()
     with _plan(np.zeros((4, 16), np.int32), 4096, 2) as h:
