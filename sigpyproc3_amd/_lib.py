@@ -236,29 +236,31 @@ def to_host(x) -> np.ndarray:
     nbytes = int(x.numel()) * x.element_size()
     if nbytes < _STAGED_MIN or not x.is_cuda:
         return x.cpu().numpy()
-    if not hasattr(_staging, "buffers"):
-        try:
-            _staging.buffers = [t.empty(STAGE_BYTES, dtype=t.uint8, pin_memory=True) for _ in range(2)]
-        except RuntimeError:  # no pinned memory to be had
-            return x.cpu().numpy()
-    src = x.contiguous().reshape(-1).view(t.uint8)
-    out = t.empty(tuple(x.shape), dtype=x.dtype)
-    dst = out.reshape(-1).view(t.uint8)
-    with t.cuda.device(x.device):
-        arrived = [t.cuda.Event(), t.cuda.Event()]
-        pieces = [(a, min(a + STAGE_BYTES, nbytes)) for a in range(0, nbytes, STAGE_BYTES)]
+    # ordinary CPU tensors under any inference mode and default device of the caller's
+    with t.inference_mode(False):
+        if not hasattr(_staging, "buffers"):
+            try:
+                _staging.buffers = [t.empty(STAGE_BYTES, dtype=t.uint8, device="cpu", pin_memory=True) for _ in range(2)]
+            except RuntimeError:  # no pinned memory to be had
+                return x.cpu().numpy()
+        out = t.empty(tuple(x.shape), dtype=x.dtype, device="cpu")
+        src = x.contiguous().reshape(-1).view(t.uint8)
+        dst = out.reshape(-1).view(t.uint8)
+        with t.cuda.device(x.device):
+            arrived = [t.cuda.Event(), t.cuda.Event()]
+            pieces = [(a, min(a + STAGE_BYTES, nbytes)) for a in range(0, nbytes, STAGE_BYTES)]
 
-        def drain(k: int) -> None:
-            a, b = pieces[k]
-            arrived[k & 1].synchronize()
-            dst[a:b].copy_(_staging.buffers[k & 1][: b - a])
+            def drain(k: int) -> None:
+                a, b = pieces[k]
+                arrived[k & 1].synchronize()
+                dst[a:b].copy_(_staging.buffers[k & 1][: b - a])
 
-        for k, (a, b) in enumerate(pieces):
-            _staging.buffers[k & 1][: b - a].copy_(src[a:b], non_blocking=True)
-            arrived[k & 1].record()
-            if k > 0:
-                drain(k - 1)
-        drain(len(pieces) - 1)
+            for k, (a, b) in enumerate(pieces):
+                _staging.buffers[k & 1][: b - a].copy_(src[a:b], non_blocking=True)
+                arrived[k & 1].record()
+                if k > 0:
+                    drain(k - 1)
+            drain(len(pieces) - 1)
     return out.numpy()
 
 
