@@ -223,7 +223,7 @@ def to_device(a: np.ndarray):
 STAGE_BYTES = 2 << 20
 _STAGED_MIN = STAGE_BYTES
 
-_staging = threading.local()  # .buffers: this thread's two pinned buffers, freed when it ends
+_staging = threading.local()  # .buffers: this thread's two pinned buffers while no call uses them
 
 
 def to_host(x) -> np.ndarray:
@@ -236,11 +236,14 @@ def to_host(x) -> np.ndarray:
     nbytes = int(x.numel()) * x.element_size()
     if nbytes < _STAGED_MIN or not x.is_cuda:
         return x.cpu().numpy()
+    # Taken out while in use: a call that interrupts this one takes its own, and one that does not
+    # end leaves none with copies still under way.
+    buffers = _staging.__dict__.pop("buffers", None)
     # ordinary CPU tensors under any inference mode and default device of the caller's
     with t.inference_mode(False):
-        if not hasattr(_staging, "buffers"):
+        if buffers is None:
             try:
-                _staging.buffers = [t.empty(STAGE_BYTES, dtype=t.uint8, device="cpu", pin_memory=True) for _ in range(2)]
+                buffers = [t.empty(STAGE_BYTES, dtype=t.uint8, device="cpu", pin_memory=True) for _ in range(2)]
             except RuntimeError:  # no pinned memory to be had
                 return x.cpu().numpy()
         out = t.empty(tuple(x.shape), dtype=x.dtype, device="cpu")
@@ -253,14 +256,15 @@ def to_host(x) -> np.ndarray:
             def drain(k: int) -> None:
                 a, b = pieces[k]
                 arrived[k & 1].synchronize()
-                dst[a:b].copy_(_staging.buffers[k & 1][: b - a])
+                dst[a:b].copy_(buffers[k & 1][: b - a])
 
             for k, (a, b) in enumerate(pieces):
-                _staging.buffers[k & 1][: b - a].copy_(src[a:b], non_blocking=True)
+                buffers[k & 1][: b - a].copy_(src[a:b], non_blocking=True)
                 arrived[k & 1].record()
                 if k > 0:
                     drain(k - 1)
             drain(len(pieces) - 1)
+    _staging.buffers = buffers
     return out.numpy()
 
 

@@ -73,3 +73,31 @@ def test_default_device(first_inside):
 
     for k, got in enumerate(_in_new_thread(work)):
         _check(got, k)
+
+
+def test_after_a_call_that_did_not_end(monkeypatch):
+    import torch
+
+    def work():
+        _lib.to_host(_series(1))
+        kept = _lib._staging.buffers
+        calls = []
+        with monkeypatch.context() as m:
+            real = torch.cuda.Event.synchronize
+
+            def interrupted(self):
+                calls.append(self)
+                if len(calls) == 2:
+                    raise KeyboardInterrupt
+                real(self)
+
+            m.setattr(torch.cuda.Event, "synchronize", interrupted)
+            with pytest.raises(KeyboardInterrupt):
+                _lib.to_host(_series(2))
+        # its copies may still be under way: another call must not fill the same buffers
+        assert getattr(_lib._staging, "buffers", None) is None
+        got = _lib.to_host(_series(5))
+        assert _lib._staging.buffers[0] is not kept[0]
+        return got
+
+    _check(_in_new_thread(work), 5)
