@@ -345,7 +345,9 @@ int spp_boxcar_mf_noalloc(const float* z, int64_t ldz, int64_t nrows, const int6
  * arithmetic; S and the box sums in float64. Each width's first maximum is taken on the
  * float64 box sums, then conv is rounded to float32 and the template-major first maximum
  * kept, so (snr, peak, widx) equal spp_boxcar_mf's except where float32 rounding makes two
- * box sums of one width equal. Rows whose good size is odd take spp_boxcar_mf's FFT path
+ * box sums of one width equal. Calls of few rows cut them into shorter blocks: for series that
+ * are not integer-valued, where the window sums round, z and with it snr can then differ from
+ * spp_running_normalise's in the last bit. Rows whose good size is odd take spp_boxcar_mf's FFT path
  * (one row at a time); a row of exactly Ng (odd) samples is refused with SPP_EINVAL.
  * Row lengths 1 <= n <= min(ldx, 2^31 - 1) and n >= the largest width; window >= 1.
  * workspace: spp_normalise_boxcar_mf_workspace_size bytes for the same row lengths and widths; one

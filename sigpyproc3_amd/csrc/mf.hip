@@ -538,8 +538,11 @@ __global__ void k_boxcar_final(const Best* __restrict__ part, int64_t nrows, int
 //
 // The running normalisation and the boxcar MF of the rows of a plane x in one pass: z never
 // leaves the block. A block takes `chb` outputs of one row (whole segments) and
-// normalises them RN_SEG at a time with k_norm's window sums and arithmetic (so z is the
-// float32 k_norm writes). Each segment's z is prefix-summed in float64, relative to the block
+// normalises them RN_SEG at a time with k_norm's arithmetic. z is the float32 k_norm writes where the
+// window sums are exact (integer-valued series) or chb is RN_CHB; otherwise the shorter blocks
+// of a call of few rows sum their first windows at other samples, and a z at a float32 rounding
+// boundary can be the neighbouring one, so that a row's S/N may depend in its last bit on how
+// many rows share the call. Each segment's z is prefix-summed in float64, relative to the block
 // start, into an LDS ring P of two segments; the box sums of the previous segment are then
 // P[u + w] - P[u]. A box reaches wmax - 1 <= MF_WMAX - 1 < RN_SEG samples into the next
 // segment, so the block normalises one segment past its chunk. The circular series wraps at
