@@ -91,7 +91,8 @@ typedef struct {
     int64_t total_samples;   /* sum of row lengths (DM-trial samples)               */
     int64_t ndm_tiles;       /* DM tiles the planner formed                         */
     int32_t max_spread;      /* largest per-channel delay spread inside a DM tile   */
-    int32_t mode;            /* field bits (4/8/16) + 32 if 32-bit lanes + 64*variant */
+    int32_t mode;            /* field bits (4/8/16) + 32 if 32-bit lanes + 64*variant (of a
+                                full-length execution, unless one was set) */
     int64_t tables_bytes;    /* leading part of the workspace holding the plan tables */
 } spp_sweep_info;
 

@@ -1,5 +1,6 @@
-// One-DM dedispersion and subbanding of a gulp, with the sub-byte unpack fused into
-// the LDS staging (the "one DM per launch" form).
+// Subbanding of a gulp, with the sub-byte unpack fused into the LDS staging, and one-DM
+// dedispersion of the gulps that the word-parallel (gulp_swar.hip) and small-block float32
+// (gulp_f32.hip) kernels do not take.
 //
 // Gulp layout: file order, [nsamps][nchans] packed nbits (1/2/4/8, bit order `big`)
 // or float32. A block owns DD_T consecutive output samples and a group of channels.
@@ -63,7 +64,7 @@ __device__ __forceinline__ int stage_extent(const int32_t* sdel, int ncand, int 
 // MODE 0: dedisperse (out[out_start + t] = sum). MODE 1: subband (out[t*nsubs + sub] += run sum).
 // Staging: the stage's channels occupy bytes [bb0, bb1) of each packed row. All threads take
 // (row, unit) elements, a unit being a dword (WIDE: rows and the stream start are 4-byte
-// aligned) or a byte, DD_LD of them in flight per thread, and unpack every sample of a unit
+// aligned; subbands only, as such rows dedisperse elsewhere) or a byte, DD_LD of them in flight per thread, and unpack every sample of a unit
 // that belongs to the stage into its tile column.
 template <int NBITS, bool BIG, int MODE, bool WIDE, int CCX, int ROWS>
 __global__ __launch_bounds__(DD_THREADS) void k_gulp_int(
@@ -448,31 +449,24 @@ int launch_int(const uint8_t* in, int nbits, int big, const int32_t* delays, con
     }
     int64_t cpg = spp::ceil_div(nchans, groups);
     int64_t ilv = 1, nchunk = 1;
-    // Dedisperse with wide groups uses groups of DD_CC channels (one stage each), numbered so
-    // that the groups of a time tile run side by side on one XCD and read each packed row line
-    // (128 bytes) from L2 once it is fetched. When the mean delay spread across one row line is
-    // at most DD_T samples, the groups that share a line read mostly the same rows; then a block
-    // takes nchunk chunks one line apart, and the ilv = line / chunk groups of a line run side
-    // by side: the same single fetch with nchunk times fewer float atomics per output. Subband
-    // otherwise keeps contiguous groups: its band partial sums are float atomics nsubs floats
-    // apart, and splitting bands across groups multiplies them.
-    // Subband takes the same interleave with chunks of whole bands (the mean band width rounded
-    // up to DD_CC channels), so a band is still summed by one block and flushed once.
+    // Subbands with wide groups: when the mean delay spread across one packed row line (128 bytes)
+    // is at most DD_T samples, the groups that share a line read mostly the same rows. Then a block
+    // takes nchunk chunks one line apart, and the ilv = line / chunk groups of a line run side by
+    // side on one XCD and read the line from L2 once it is fetched. A chunk is whole bands (the mean
+    // band width rounded up to DD_CC channels), so a band is still summed by one block and flushed
+    // once. Otherwise groups are contiguous: band partial sums are float atomics nsubs floats
+    // apart, and splitting bands across groups multiplies them. (Dedispersion in wide groups is
+    // the word-parallel kernel's.)
     const int64_t line_ch = 1024 / nbits;
     const int64_t line_spread = (nsamps - nout) * line_ch / nchans;
-    const int64_t chunk = MODE == 0 ? DD_CC
-                                    : spp::ceil_div(spp::ceil_div(nchans, std::max<int64_t>(1, nsubs)),
-                                                    int64_t(DD_CC)) * DD_CC;
-    const bool wide_groups = exact && cpg >= DD_CC && nchans >= line_ch;
+    const int64_t chunk = spp::ceil_div(spp::ceil_div(nchans, std::max<int64_t>(1, nsubs)), int64_t(DD_CC)) * DD_CC;
+    const bool wide_groups = MODE == 1 && exact && cpg >= DD_CC && nchans >= line_ch;
     if (wide_groups && line_spread <= DD_T && line_ch % chunk == 0) {
         cpg = chunk;
         ilv = line_ch / chunk;
         const int64_t hgroups = std::max<int64_t>(1, spp::ceil_div(groups, ilv));
         nchunk = spp::ceil_div(nchans, line_ch * hgroups);
         groups = ilv * spp::ceil_div(nchans, line_ch * nchunk);
-    } else if (MODE == 0 && wide_groups) {
-        cpg = DD_CC;
-        groups = spp::ceil_div(nchans, int64_t(DD_CC));
     } else {
         // Group starts on multiples of 64 channels keep full stages dword-aligned (a power-of-two
         // unit count per stage); narrow groups on multiples of 8.
@@ -495,13 +489,14 @@ int launch_int(const uint8_t* in, int nbits, int big, const int32_t* delays, con
     hipLaunchKernelGGL((k_gulp_int<NB, BG, MODE, W, CX, R>), grid, dim3(DD_THREADS), 0, st, in, delays, cts, \
                        out, nchans, nsamps, nout, out_start, row_bytes, cpg, use_atomic, nsubs, out_size, groups, \
                        nblocks, ilv, nchunk)
+    constexpr bool W = MODE == 1;  // dword units exist for subbands only
 #define SPP_GULP_LAUNCH(NB, BG)                            \
-    if (wide && narrow)                                    \
-        SPP_GULP_ONE(NB, BG, true, 16, DD_ROWS);           \
-    else if (wide && low)                                  \
-        SPP_GULP_ONE(NB, BG, true, DD_CC, DD_ROWS_LOW);    \
-    else if (wide)                                         \
-        SPP_GULP_ONE(NB, BG, true, DD_CC, DD_ROWS);        \
+    if (W && wide && narrow)                               \
+        SPP_GULP_ONE(NB, BG, W, 16, DD_ROWS);              \
+    else if (W && wide && low)                             \
+        SPP_GULP_ONE(NB, BG, W, DD_CC, DD_ROWS_LOW);       \
+    else if (W && wide)                                    \
+        SPP_GULP_ONE(NB, BG, W, DD_CC, DD_ROWS);           \
     else if (narrow)                                       \
         SPP_GULP_ONE(NB, BG, false, 16, DD_ROWS);          \
     else if (low)                                          \

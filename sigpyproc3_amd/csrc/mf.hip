@@ -125,17 +125,6 @@ __device__ __forceinline__ int32_t wave_min(int32_t v) {
     return __builtin_amdgcn_readlane(v, 63);
 }
 
-// The largest unsigned int across the wave, in every lane.
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xf, 0xf, false)));
-    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xf, 0xf, false)));
-    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xf, 0xf, false)));
-    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x118, 0xf, 0xf, false)));
-    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xa, 0xf, false)));
-    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xc, 0xf, false)));
-    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
-}
-
 // The value of the previous lane (0.0 in lane 0): wave_shr:1.
 __device__ __forceinline__ double wave_prev(double v) { return dpp_move<0x138, 0xf>(v); }
 
