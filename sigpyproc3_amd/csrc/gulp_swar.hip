@@ -542,13 +542,15 @@ bool gulp_swar_applies(int nbits, bool aligned, int64_t nchans, int64_t nout, in
     if (aligned || nbits >= 4) return true;
     // 1/2-bit rows that are not whole dwords: a block covers four times the outputs and up to eight
     // times the channels of the byte-staged kernel's (k_gulp_int), so a short gulp leaves it few
-    // blocks, and a stage whose delays spread takes a pass for every 450 rows of them. This kernel
-    // against that (us), 1-bit: 336 channels x 20011 17 / 10, 72 x 262144 with 20000 rows of spread
-    // 202 / 86, 1000 x 262144 49 / 201; 2-bit: 36 x 262144 with 20000 135 / 52, 1004 x 262144 58 / 203.
+    // blocks, and a stage whose delays spread takes a pass for every 450 rows of them. So either
+    // blocks enough, or samples enough that the other's issue slots fill. This kernel against that
+    // (us), 1-bit: 336 channels x 20011 17 / 10, x 65536 17 / 20, 72 x 262144 with 20000 rows of spread
+    // 202 / 86, 1000 x 262144 49 / 201; 2-bit: 132 x 65536 14 / 10, 36 x 262144 with 20000 135 / 52,
+    // 1004 x 262144 58 / 203.
     const int64_t chunk = gulp_swar_stage_channels(nbits, GulpForm::normal);
     const int64_t blocks = ceil_div(nout, gulp_swar_tile(nbits)) * ceil_div(nchans, chunk);
     const int64_t spread = max_delay * std::min(chunk, nchans) / nchans;
-    return blocks * 2500 >= 100 * (2500 + spread);
+    return blocks * 2500 >= 100 * (2500 + spread) || nout * nchans / (1500 + spread) >= 14000000 / 1500;
 }
 
 int launch_gulp_swar(const uint8_t* in, int nbits, bool big, const int32_t* delays, float* out, int64_t nchans,

@@ -24,6 +24,8 @@ def _word_parallel(nbits, nchans, nsamps, md, aligned=False):
     [
         # times measured in the word-parallel and in the byte-staged kernel, in us
         (1, 336, 20011, 500, False),      # 17, 9
+        (1, 336, 65536, 500, True),       # 17, 20
+        (2, 132, 65536, 0, False),        # 14, 10
         (1, 72, 262144, 20000, False),    # 202, 86
         (1, 1040, 4096, 0, False),        # 17, 10
         (1, 1000, 262144, 5000, True),    # 49, 201
