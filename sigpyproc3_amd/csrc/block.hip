@@ -80,9 +80,9 @@ __global__ __launch_bounds__(RB_THREADS) void k_roll_rows4(const float* __restri
 // Measured on 1024 channels x 8192 samples, 512 DM rows: 2436 -> 618 us (4.3e9 adds; the LDS
 // reads alone take 220 at 128 bytes per clock and CU, the rest is the wait of each 5-channel
 // stage). Windows of 128 spare samples and 8 channels run 528 there but leave 2000 channels x
-// 16384, 128 rows (offsets up to 450 apart) to memory. Channels added from memory have a stage's 32
-// loads in flight: 1024 x 65536, 32 rows spread over 30000 samples, 1042 us (1587 with a thread per
-// output and one load in flight).
+// 16384, 128 rows (offsets up to 450 apart) to memory. Where most channels are added from memory:
+// 1024 x 65536, 32 rows spread over 30000 samples, 1230 us (1587 with a thread per output and one load
+// in flight, 2380 in a tile with one in flight).
 constexpr int DT_D = 8;         // DM rows per block
 constexpr int DT_K = 4;         // samples per thread
 constexpr int DT_CC = 5;        // channels per stage
@@ -176,11 +176,14 @@ __global__ __launch_bounds__(RB_THREADS) void k_dmt(const float* __restrict__ in
 #pragma unroll
             for (int j = 0; j < K; ++j) acc[r][j] = acc[r][j] + v[r][j];
     };
-    int td[K];  // the thread's samples; those past the last output repeat it
-#pragma unroll
-    for (int j = 0; j < K; ++j) td[j] = min(t0 + tid + RB_THREADS * j, out_cols - 1);
+    // A channel without a window: a row's loads at a time, the rows' waits at the end. (The empty asm
+    // keeps the compiler from mixing the rows: with all 32 loads in one group the staged sums get fewer
+    // registers, 630 us instead of 587 at 1024 x 8192, 512 rows, for 1002 instead of 1230 at the spread rows named above.)
     auto add_direct = [&](int64_t c) {
         const float* __restrict__ row = in + c * ncols;
+        int td[K];  // the thread's samples; those past the last output repeat it
+#pragma unroll
+        for (int j = 0; j < K; ++j) td[j] = min(t0 + tid + RB_THREADS * j, out_cols - 1);
         float v[DT_D][K];
 #pragma unroll
         for (int r = 0; r < DT_D; ++r) {
@@ -190,11 +193,13 @@ __global__ __launch_bounds__(RB_THREADS) void k_dmt(const float* __restrict__ in
                 const int col = o + td[j];
                 v[r][j] = row[col >= ncols ? col - ncols : col];
             }
+            asm volatile("");
         }
 #pragma unroll
         for (int r = 0; r < DT_D; ++r)
 #pragma unroll
             for (int j = 0; j < K; ++j) acc[r][j] = acc[r][j] + v[r][j];
+        asm volatile("");
     };
     for (int64_t c0 = 0; c0 < nchans; c0 += DT_PLAN) {
         bool mine = true;
