@@ -402,11 +402,9 @@ int launch_swar(const uint8_t* in, int nbits, int big, const int32_t* delays, fl
     int64_t ilv = 1, nchunk = 1;
     const int64_t line_ch = 1024 / nbits;  // channels in a 128-byte row line
     const int64_t line_spread = (nsamps - nout) * line_ch / nchans;
-    // Also for rows that are not whole lines (neighbouring chunks still share most lines): 8-bit 1000
-    // channels x 200000 samples 200 us in contiguous groups, 86 with the line's groups side by side;
-    // not for 4-bit ones (1000 x 200000: 62 / 68).
-    const bool wide_groups = exact && cpg >= chunk && nchans >= line_ch && (nbits != 4 || nchans % line_ch == 0);
-    if (wide_groups && line_spread <= T) {
+    const bool near = line_spread <= T;
+    const bool wide_groups = exact && cpg >= chunk && spp::gulp_swar_by_lines(nbits, nchans, nout, nsamps - nout);
+    if (wide_groups && near) {
         cpg = chunk;
         ilv = line_ch / chunk;
         const int64_t hgroups = std::max<int64_t>(1, spp::ceil_div(groups, ilv));

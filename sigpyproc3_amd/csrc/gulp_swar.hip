@@ -553,6 +553,23 @@ bool gulp_swar_applies(int nbits, bool aligned, int64_t nchans, int64_t nout, in
     return blocks * 2500 >= 100 * (2500 + spread) || nout * nchans / (1500 + spread) >= 14000000 / 1500;
 }
 
+bool gulp_swar_by_lines(int nbits, int64_t nchans, int64_t nout, int64_t max_delay) {
+    const int64_t line_ch = 1024 / nbits;  // channels in a 128-byte row line
+    if (nchans < line_ch) return false;
+    if (nchans % line_ch == 0) return true;
+    // Rows that are not whole lines (neighbouring chunks still share most lines) take a line's groups
+    // side by side, or 8-bit ones whose delays spread a group per chunk, only in gulps of many bytes:
+    // below, the groups of a cut line are blocks of little work. Measured, so against contiguous groups
+    // (us): 8-bit 1000 channels x 200000 86 / 200, 160 x 524288 (84 MB) 40 / 48, x 262144 26 / 21; 2-bit
+    // 896 x 524288 (117 MB) 57 / 66, 640 x 524288 (84 MB) 58 / 49; 1-bit 2560 x 524288 (168 MB) 113 / 132,
+    // 2176 (143 MB) 115 / 107; with delays of 8000 1-bit 2304 x 262144 (75 MB) 67 / 80, 8-bit 192 x
+    // 262144 (50 MB) 40 / 37. Not for 4-bit ones (1000 x 200000: 68 / 62).
+    if (nbits == 4) return false;
+    const bool near = max_delay * line_ch / nchans <= gulp_swar_tile(nbits);
+    const int64_t least = near ? (nbits == 8 ? 60 : (nbits == 2 ? 100 : 150)) : (nbits == 8 ? 75 : 0);  // MB
+    return nchans * nbits / 8 * nout >= least * 1000000;
+}
+
 int launch_gulp_swar(const uint8_t* in, int nbits, bool big, const int32_t* delays, float* out, int64_t nchans,
                      int64_t nsamps, int64_t nout, int64_t out_start, int64_t row_bytes, int64_t chans_per_group,
                      int64_t groups, int64_t ilv, int64_t nchunk, int use_atomic, GulpForm form, hipStream_t st) {

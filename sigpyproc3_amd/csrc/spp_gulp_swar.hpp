@@ -25,6 +25,10 @@ int launch_gulp_swar(const uint8_t* in, int nbits, bool big, const int32_t* dela
                      int64_t nsamps, int64_t nout, int64_t out_start, int64_t row_bytes, int64_t chans_per_group,
                      int64_t groups, int64_t ilv, int64_t nchunk, int use_atomic, GulpForm form, hipStream_t st);
 
+// True when channel groups follow the 128-byte lines of the rows (one stage's channels a chunk), false
+// when they are contiguous.
+bool gulp_swar_by_lines(int nbits, int64_t nchans, int64_t nout, int64_t max_delay);
+
 // Outputs per block for nbits (the time tile).
 int64_t gulp_swar_tile(int nbits);
 

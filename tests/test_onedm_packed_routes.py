@@ -46,6 +46,63 @@ def test_rule(nbits, nchans, nsamps, md, word):
         assert _word_parallel(nbits, nchans, nsamps, md, aligned=True)
 
 
+def _by_lines(nbits, nchans, nsamps, md):
+    fn = _lib.load()._ZN3spp18gulp_swar_by_linesEilll  # spp::gulp_swar_by_lines(nbits, nchans, nout, max_delay)
+    fn.restype = ctypes.c_bool
+    fn.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3
+    return fn(nbits, nchans, nsamps - md, md)
+
+
+@pytest.mark.parametrize(
+    ("nbits", "nchans", "nsamps", "md", "lines"),
+    [
+        # times measured by lines and in contiguous groups, in us
+        (8, 1024, 65536, 2000, True),     # whole lines
+        (8, 1000, 200000, 5000, True),    # 86, 200
+        (8, 160, 524288, 100, True),      # 40, 48
+        (8, 160, 262144, 100, False),     # 26, 21
+        (8, 192, 262144, 8000, False),    # 40, 37
+        (8, 124, 1 << 20, 0, False),      # less than a line
+        (4, 1000, 200000, 5000, False),   # 68, 62
+        (2, 896, 524288, 100, True),      # 57, 66
+        (2, 640, 524288, 100, False),     # 58, 49
+        (2, 1152, 262144, 8000, True),    # 53, 70
+        (1, 2560, 524288, 100, True),     # 113, 132
+        (1, 2176, 524288, 100, False),    # 115, 107
+        (1, 2304, 262144, 8000, True),    # 67, 80
+    ],
+)
+def test_line_rule(nbits, nchans, nsamps, md, lines):
+    assert _by_lines(nbits, nchans, nsamps, md) == lines
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(("nbits", "nchans", "nsamps", "hi", "lines"), [
+    (8, 160, 380000, 100, True), (8, 160, 100000, 100, False), (8, 192, 400000, 9000, True), (8, 300, 100003, 9000, False),
+    (2, 640, 640000, 900, True), (2, 640, 100000, 900, False), (2, 1152, 100000, 8000, True), (1, 1312, 200000, 3000, True),
+    (1, 1312, 200000, 300, False)])
+def test_cut_lines(nbits, nchans, nsamps, hi, lines):
+    import torch
+
+    assert _by_lines(nbits, nchans, nsamps, hi) == lines
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(nchans)
+    packed = torch.randint(0, 256, (nsamps, nchans * nbits // 8), generator=gen, device="cuda", dtype=torch.uint8)
+    delays = np.round(np.linspace(0, 1, nchans) ** 2 * hi).astype(np.int32)
+    per = 8 // nbits
+    want = torch.zeros(nsamps - hi, dtype=torch.int64, device="cuda")
+    for c in range(nchans):
+        byte = packed[int(delays[c]) : int(delays[c]) + nsamps - hi, c // per]
+        want += (byte >> (8 - (c % per + 1) * nbits)) & ((1 << nbits) - 1)  # big bit order
+    out = torch.full((nsamps - hi + 2,), -1.0, device="cuda")
+    d = _lib.to_device(delays)
+    _lib.call("spp_dedisperse", _lib.ptr(packed), nbits, 1, nchans, nsamps, _lib.ptr(d), hi, _lib.ptr(out), 1,
+              _lib.stream_handle())
+    got = out.cpu().numpy()
+    assert got[0] == -1 and got[-1] == -1
+    np.testing.assert_array_equal(got[1:-1], want.cpu().numpy().astype(np.float32))
+
+
 def _samples(packed_rows, nbits, nchans, big):
     per = 8 // nbits
     shifts = [(8 - (k + 1) * nbits) if big else k * nbits for k in range(per)]
