@@ -1,5 +1,6 @@
-"""spp_dmt where its launch takes the tiled kernel: windows that wrap, do not fit, or come from
-rows of very different offsets. Channels are added in order in float32, so equality is exact."""
+"""spp_dmt on grids about as large as the tiled kernel takes: windows that wrap, do not fit, or come
+from rows of very different offsets (test_dmt_routes.py asserts which calls take tiles). Channels are
+added in order in float32, so equality is exact."""
 
 from __future__ import annotations
 

@@ -2,11 +2,13 @@
 
 It must give spp_boxcar_mf(spp_running_normalise(x)) -- the two-pass GPU form, itself
 pinned against the float64 oracle in test_gpu_parity.py and test_gpu_mf_odd.py -- with the
-same (peak, width) and snr within rel 2e-6 (only the order of the float64 sum S differs),
-and the oracle's answer directly on sampled rows. Row lengths cover: shorter than one
-2048-sample segment, segment and 32768-sample chunk edges, boxes that cross the row end
-(the circular wrap), good sizes far above n (z[0, Ng - n) counted twice in S), odd good
-sizes (the FFT path), the 12- and 32-width kernels, odd windows and unaligned rows.
+same (peak, width) and snr within rel 2e-6 (the float64 sum S is added in another order, and
+z of non-integer series may round differently where the blocks are shorter than the two-pass
+form's), and the oracle's answer directly on sampled rows. Row lengths cover: shorter than one
+2048-sample segment, segment and block edges of the short blocks that few rows take (longer
+ones in test_gpu_mf_chunks.py), boxes that cross the row end (the circular wrap), good sizes
+far above n (z[0, Ng - n) counted twice in S), odd good sizes (the FFT path), 1 to 32 widths,
+odd windows and unaligned rows.
 """
 
 from __future__ import annotations
@@ -136,7 +138,7 @@ def test_sweep_result_matched_filter_uses_one_pass():
 @pytest.mark.parametrize("nwidths", [1, 2, 13, 31, 32])
 @pytest.mark.parametrize("nrows", [1, 40])
 def test_fused_block_lengths_and_width_counts(nrows, nwidths):
-    """Few rows take shorter blocks (2 to 16 segments); any number of widths is one kernel."""
+    """Few rows take the shortest blocks (2 segments); any number of widths is one kernel."""
     rng = np.random.default_rng(100 * nrows + nwidths)
     widths = sorted(rng.choice(np.arange(1, 513), nwidths, replace=False).tolist())
     n = 5 * 2048 + 17 if nrows == 1 else 16 * 2048 * 3 - 1

@@ -1,5 +1,6 @@
-"""spp_subband on 8-bit gulps whose launch takes the whole-band kernel: band maps, delays and
-sizes at the edges of its stages. Sums are integers below 2^24, so equality is exact."""
+"""spp_subband on 8-bit gulps of many outputs: band maps, delays and sizes at the edges of the
+whole-band kernel's stages, some of which the byte-staged kernel takes (test_subband8_bands.py asserts
+which calls take which). Sums are integers below 2^24, so equality is exact."""
 
 from __future__ import annotations
 

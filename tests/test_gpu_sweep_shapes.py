@@ -1,5 +1,5 @@
-"""The block shape an execution takes by its size: both sides of every line of the rule, on plans
-whose shape nobody set, against the C oracle (integer sums, so bit for bit)."""
+"""Executions of plans whose shape nobody set, of one to 16385 blocks and with few rows per tile, against
+the C oracle (integer sums, so bit for bit). test_sweep_shape_rule.py asserts the shapes themselves."""
 
 import numpy as np
 import pytest
