@@ -239,31 +239,30 @@ def to_host(x) -> np.ndarray:
     # Taken out while in use: a call that interrupts this one takes its own, and one that does not
     # end leaves none with copies still under way.
     buffers = _staging.__dict__.pop("buffers", None)
-    # ordinary CPU tensors under any inference mode and default device of the caller's
-    with t.inference_mode(False):
-        if buffers is None:
-            try:
+    if buffers is None:
+        try:
+            with t.inference_mode(False):  # they outlive the caller's mode
                 buffers = [t.empty(STAGE_BYTES, dtype=t.uint8, device="cpu", pin_memory=True) for _ in range(2)]
-            except RuntimeError:  # no pinned memory to be had
-                return x.cpu().numpy()
-        out = t.empty(tuple(x.shape), dtype=x.dtype, device="cpu")
-        src = x.contiguous().reshape(-1).view(t.uint8)
-        dst = out.reshape(-1).view(t.uint8)
-        with t.cuda.device(x.device):
-            arrived = [t.cuda.Event(), t.cuda.Event()]
-            pieces = [(a, min(a + STAGE_BYTES, nbytes)) for a in range(0, nbytes, STAGE_BYTES)]
+        except RuntimeError:  # no pinned memory to be had
+            return x.cpu().numpy()
+    src = x.contiguous().reshape(-1).view(t.uint8)
+    out = t.empty(tuple(x.shape), dtype=x.dtype, device="cpu")
+    dst = out.reshape(-1).view(t.uint8)
+    with t.cuda.device(x.device):
+        arrived = [t.cuda.Event(), t.cuda.Event()]
+        pieces = [(a, min(a + STAGE_BYTES, nbytes)) for a in range(0, nbytes, STAGE_BYTES)]
 
-            def drain(k: int) -> None:
-                a, b = pieces[k]
-                arrived[k & 1].synchronize()
-                dst[a:b].copy_(buffers[k & 1][: b - a])
+        def drain(k: int) -> None:
+            a, b = pieces[k]
+            arrived[k & 1].synchronize()
+            dst[a:b].copy_(buffers[k & 1][: b - a])
 
-            for k, (a, b) in enumerate(pieces):
-                buffers[k & 1][: b - a].copy_(src[a:b], non_blocking=True)
-                arrived[k & 1].record()
-                if k > 0:
-                    drain(k - 1)
-            drain(len(pieces) - 1)
+        for k, (a, b) in enumerate(pieces):
+            buffers[k & 1][: b - a].copy_(src[a:b], non_blocking=True)
+            arrived[k & 1].record()
+            if k > 0:
+                drain(k - 1)
+        drain(len(pieces) - 1)
     _staging.buffers = buffers
     return out.numpy()
 
