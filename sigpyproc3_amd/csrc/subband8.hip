@@ -37,7 +37,6 @@ constexpr int SB_Q = 4;                    // 16-channel groups per stage
 constexpr int SB_CH = 16 * SB_Q;           // channels per stage
 constexpr int SB_NRB = SB_T / 4 + 1;       // series dwords of a channel: its outputs' and the funnel's upper one
 constexpr int SB_PITCH = SB_NRB + 2;       // a spare dword, and odd: the groups a wave writes fall 16 banks apart
-constexpr int SB_WIDE = 256;               // channels of a band that one block sums at most
 constexpr int SB_UNITS = 6;                // units of the next stage each thread loads ahead
 // Word 3 of a raw buffer resource on gfx9-family GPUs: 32-bit data format, no swizzle.
 constexpr int kBufferFlags = 0x00020000;
@@ -65,7 +64,7 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
                                                          float* __restrict__ out, int64_t nchans, int64_t nsamps,
                                                          int64_t nout, int64_t nsubs, int64_t out_size,
                                                          int64_t chans_per_group, int64_t ngroups,
-                                                         int64_t nblocks) {
+                                                         int64_t nblocks, int widest) {
     __shared__ uint32_t series[SB_CH * SB_PITCH];
     __shared__ int32_t sdel[2][SB_CH], ssub[2][SB_CH], sshift[2][SB_CH];
     __shared__ int32_t gmin[2][SB_Q], gmax[2][SB_Q];
@@ -82,11 +81,10 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
     const int64_t ce = min(nchans, cb + chans_per_group);
 
     // Bands of consecutive channels (a non-decreasing or non-increasing map)? Then this block's
-    // channels are the bands that start in [cb, ce), to their ends. A band of more than SB_WIDE
+    // channels are the bands that start in [cb, ce), to their ends. A band of more than `widest`
     // channels is not one block's chain of stages: the blocks whose ranges it covers each add
     // their part of it. 1024 channels x 131072, one band of 961 among 63 of one channel: 197 us in
-    // one block, 175 shared; 4096 x 16384, one of 3969 among 127: 463 and 90; four of 200: 114, and
-    // 152 if bands of more than 128 are shared.
+    // one block, 175 shared; 4096 x 16384, one of 3969 among 127: 463 and 90.
     bool valid = true, up = true, down = true;
     int start_cb = 0, after_cb = static_cast<int>(nchans);  // band starts: last up to cb, first past it
     int start_ce = 0, after_ce = static_cast<int>(nchans);  // and about ce
@@ -139,8 +137,8 @@ __global__ __launch_bounds__(SB_THREADS) void k_subband8(const uint8_t* __restri
     const int tail0 = __builtin_amdgcn_readfirstlane(bd.z), tail1 = __builtin_amdgcn_readfirstlane(bd.w);
     const bool head = sorted && head0 < cb;                // the block's first channel is in a band before it,
     const bool tail = sorted && ce < nchans && tail0 < ce;  // its last one in a band that goes on
-    bool shared_head = head && head1 - head0 > SB_WIDE;
-    const bool shared_tail = tail && tail1 - tail0 > SB_WIDE;
+    bool shared_head = head && head1 - head0 > widest;
+    const bool shared_tail = tail && tail1 - tail0 > widest;
     const int64_t lo = head && !shared_head ? head1 : cb;
     const int64_t hi = tail && !shared_tail ? tail1 : ce;
     if (lo >= ce) return;  // one band of another block
@@ -420,8 +418,14 @@ bool subband8_applies(const void* in, int64_t nchans, int64_t nsamps, int64_t no
     // spread, 8 bands x 32768 outputs: 23 / 12.5 (64 channels), 22.5 / 33 (512 channels, 32 groups);
     // 16 x 32768 25 / 31. With 8192 rows of spread: 8 x 98304 82 / 51, 32 x 98304 97 / 162, 8 x 458752
     // 117 / 236; with 16384: 8 x 131072 (32 channels) 105 / 46, 8 x 491520 119 / 121.
+    // With fewer than 8 bands there are few atomics, and the other kernel is slow only where delays
+    // spread (64 channels in one band x 524288 19 / 37 at 200 rows, 20 / 15 at none; 128 in two x 131072
+    // 18 / 16 at none, 29 / 49 at 1500) or bands are narrow (64 in 4 x 524288 24 / 37, x 131072 20 / 13).
     const int64_t groups = std::min(ceil_div(int64_t(8) * device_cu_count(), ceil_div(nout, int64_t(512))), ceil_div(nchans, int64_t(16)));
     const int64_t spread = (nsamps - nout) * 16 / std::max<int64_t>(nchans, 16);
+    if (nsubs < 8)
+        return (spread >= 128 && nout * nchans >= 12000000) ||
+               (nsubs >= 4 && nchans <= 64 && nout * nsubs >= 700000 + 110 * spread);
     return nout * std::max(nsubs, groups) >= 300000 + 110 * spread;
 }
 
@@ -434,9 +438,13 @@ int launch_subband8(const uint8_t* in, const int32_t* delays, const int32_t* cha
     const int64_t groups = ceil_div(nchans, cpg);
     const int64_t nblocks = bx * groups;
     SPP_REQUIRE(nblocks <= 0x7ffffff0LL, "gulp too long");
+    // Few time tiles, or bands, leave CUs idle while one block sums a wide band: 512 channels with a band
+    // of 250 x 40000 50 us in one block, 33 shared; four of 200 in 1024 channels 56 and 52, but x 131072
+    // 101 and 136; one of 200 in 228 channels and four bands x 262144 110 and 83.
+    const int widest = bx <= 40 || nsubs < 8 ? 128 : 256;
     hipLaunchKernelGGL(k_subband8, dim3(static_cast<unsigned>(ceil_div(nblocks, int64_t(8)) * 8)), dim3(SB_THREADS),
                        0, st, in, delays, chan_to_sub, out, nchans, nsamps, nout, nsubs, out_size, cpg, groups,
-                       nblocks);
+                       nblocks, widest);
     SPP_LAUNCHED("k_subband8");
     return SPP_OK;
 }

@@ -36,6 +36,13 @@ def _applies(nchans, nsamps, md, nsubs, address=4096):
         (4096, 65536, 2500, 32, True),     # 128-channel bands
         (4096, 65536, 2500, 16, False),    # 256-channel bands
         (1026, 131072, 0, 64, False),      # rows that are not whole dwords
+        (64, 524288, 0, 1, False),         # 20, 15: few bands
+        (64, 524288, 800, 1, True),        # 19, 37
+        (64, 131072, 800, 2, False),       # 18, 10
+        (128, 131072, 12000, 2, True),     # 29, 49
+        (64, 131072, 0, 4, False),         # 20, 13
+        (64, 524288, 0, 4, True),          # 24, 37
+        (24, 131072, 0, 6, True),          # 16, 21
     ],
 )
 def test_rule(nchans, nsamps, md, nsubs, whole):
@@ -97,6 +104,16 @@ def test_band_widths(name, falling):
     assert len(bands) == nchans and bands.max() < nsubs
     delays = np.round(np.linspace(0, 300, nchans)).astype(np.int32)
     _compare(nchans, nsubs, 20000, delays, bands[::-1] if falling else bands, cut=7 if falling else 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("widths", [(10, 128, 30, 129, *([8] * 40), 23), (250, 250, *([4] * 35))])
+def test_widest_band_of_one_block_by_gulp_length(widths):
+    """Bands of 129 to 256 channels are shared in short gulps only."""
+    bands = _runs(*widths)
+    delays = np.round(np.linspace(0, 300, len(bands))).astype(np.int32)
+    for nsamps in (20000, 60000):
+        _compare(len(bands), 48, nsamps, delays, bands)
 
 
 @pytest.mark.gpu
