@@ -346,7 +346,7 @@ def bench_batch(args) -> int:
     batch = SweepBatch(plans, g_budget=budget)
     batch.bind(packed, planes)
     log(f"batch: {batch.info.rounds} rounds of {batch.info.pool_bytes / 2**30:.1f} GiB G pools, "
-        f"{batch.info.build_items} stage-1 and {batch.info.sweep_items} stage-2 items")
+        f"{batch.info.build_items} stage-1 units (128 words x 32 bytes) and {batch.info.sweep_items} stage-2 items")
     tune_ms = None
     if args.variant >= 0:
         batch.set_shape(args.variant, 1)
@@ -411,7 +411,7 @@ def bench_batch(args) -> int:
                                "U[500, 3000]; float32 DM x time planes (all resident)",
                    "instances": desc, "dm_trial_samples": total,
                    "g_budget_bytes": int(budget), "rounds": int(info.rounds),
-                   "pool_bytes": int(info.pool_bytes), "stage1_items": int(info.build_items),
+                   "pool_bytes": int(info.pool_bytes), "stage1_units": int(info.build_items),
                    "stage2_items": int(info.sweep_items)},
         "batch_shape": {"shape": shape[0], "time_tiles_per_item": shape[1],
                         "dm_rows_per_item": int(info.dm_rows_per_item),

@@ -165,7 +165,8 @@ typedef struct spp_batch spp_batch;
 typedef struct {
     int64_t workspace_bytes;     /* device workspace the caller must provide            */
     int64_t pool_bytes;          /* bytes of one stage-1 pool                           */
-    int64_t build_items;         /* stage-1 work, in units of 128 words x 32 packed bytes */
+    int64_t build_items;         /* stage-1 work, in units of 128 words x 32 packed bytes (an item of
+                                    the queue is one unit, or two in shapes of 16 channels) */
     int64_t sweep_items;         /* stage-2 queue items                                 */
     int32_t rounds;              /* rounds the G budget needs (1: all copies resident)   */
     int32_t segments;            /* queue segments (2 per round)                        */
